@@ -1922,6 +1922,7 @@ int potential_rec_impl(msx_ctx ctx, const msx_atom* atoms, int64_t natoms, const
     ra.ny = ny;
     ra.nmult = nmult;
     ra.mmult = mmult;
+    ra.has_ads = ads != nullptr;
     ra.curves = nullptr;
     ra.npoints = 0;
     ra.dds = 1.0;

@@ -210,6 +210,7 @@ struct RecArgs {
     double2* out;          // V(g) of slices kz0 .. kz0+nslices-1: [slice][nx][ny]
     double A, B, cg, inv_area;  // reciprocal lengths 1/(a sin gam), 1/(b sin gam); cos gam; 1/area
     int nx, ny, nmult, mmult, kz0;
+    int has_ads;  // some segment has an absorption factor
     // tabulated curves (instead of Doyle-Turner): [type][npoints] at |g|/2 = i*dds,
     // already including the Debye-Waller factor and 1/area; seg.Z = type
     const double* curves;

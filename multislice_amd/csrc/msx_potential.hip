@@ -399,22 +399,9 @@ hipError_t launch_displace(const AtomIO* in, long long n, const double* u_rms, u
 //   F_s(g) = sum_j a_j exp(-(b_j + B_s) |g|^2/4) / area   (Doyle-Turner, Debye-Waller B),
 // at the reflections whose grid index h*nmult (k*mmult) is below n/2 in
 // magnitude; every other coefficient (Nyquist, non-multiples) is 0.
-// One 16x16 tile of reflections per block.  The phase factor of an atom is
-// separable, exp(-2 pi i h x_f) exp(-2 pi i k y_f): per chunk of 8 atoms the
-// block evaluates the 16 + 16 factors of its tile row and column once (one
-// FP64 sincospi per thread, argument reduced to [-1/2, 1/2]) into LDS, and
-// each thread forms the 8 products for its reflection (4 FP64 FMA each).
-__device__ __forceinline__ bool refl_index(int i, int n, int mult, int* h) {
-    const int half = n / 2;
-    if (i < half) {
-        *h = i / mult;
-        return i % mult == 0;
-    }
-    const int j = n - i;
-    *h = -(j / mult);
-    return i > half && j % mult == 0;
-}
-
+// The phase factor of an atom is separable, exp(-2 pi i h x_f) exp(-2 pi i k
+// y_f), so the sum over a species' atoms is a complex matrix product (rows h,
+// columns k, inner dimension the atoms) and runs on the FP64 matrix cores.
 // linear interpolation in a curve table, nothing past the end (Pot_RS.cpp:40-46,
 // Pot_rec_curve_DW.cpp:38-44)
 __device__ __forceinline__ bool curve_at(const double* c, int npoints, double u, double* out) {
@@ -425,66 +412,161 @@ __device__ __forceinline__ bool curve_at(const double* c, int npoints, double u,
     return true;
 }
 
-__global__ __launch_bounds__(256) void rec_sf_kernel(RecArgs p) {
-    __shared__ double2 ph[8][32];
-    const int ty = threadIdx.x & 15, tx = threadIdx.x >> 4;
-    const int iy = blockIdx.x * 16 + ty, ix = blockIdx.y * 16 + tx;
+// Reflections are enumerated densely whatever nmult and mmult: rows h = 0 ..
+// rec_count(nx, nmult) - 1, columns k = -(K - 1) .. K - 1 with K =
+// rec_count(ny, mmult), and a last column for the zeros at Nyquist.
+// A work-group takes kRecRows rows by kRecCols columns of one slice, each of
+// its 4 wavefronts one 16-row by 32-column part (two 16x16x4 FP64 MFMA tiles,
+// real and imaginary sums).  Only rows h >= 0 are summed: occupancies are
+// real, so S(-h, -k) is the conjugate of S(h, k) and F_s(-g) = F_s(g), and
+// each reflection writes its opposite too (with absorption factors the two
+// differ in the sign of the ads S terms, kept in sums of their own: ADS).
+// Per chunk of kRecAtoms atoms the phase factors of the tile's rows and
+// columns go to LDS as products of a factor per group of 8 and one of 8 steps
+// (28 sincospi per atom instead of 96; arguments reduced to [-1/2, 1/2]), and
+// on orthogonal cells the scattering factor is a product of a row and a
+// column exponential (1.5 exponentials per thread and species instead of 32).
+// Without these the vector unit, not the matrix cores, was the bound: 460 us
+// for 512^2, 20 slices of 360 atoms in two or three species; 258 us with
+// them, against 1095 us for one reflection per thread and vector FMAs.
+typedef double d4 __attribute__((ext_vector_type(4)));
+constexpr int kRecRows = 32, kRecCols = 64, kRecAtoms = 16;
+constexpr int kRecGroups = (kRecRows + kRecCols) / 8;  // groups of 8 rows, then of 8 columns
+__host__ __device__ inline int rec_count(int n, int mult) { return (n / 2 + mult - 1) / mult; }
+
+// SEP: Doyle-Turner on an orthogonal cell, where the scattering factor
+// separates; an instantiation of its own, since the other one's 8 inlined
+// exponentials hold 205 registers (two waves per SIMD).
+template <bool ADS, bool SEP>
+__global__ __launch_bounds__(256, SEP && !ADS ? 3 : 2) void rec_sf_kernel(RecArgs p) {
+    __shared__ double2 ph[kRecAtoms][kRecRows + kRecCols];
+    // per atom: the groups' first factors, then 8 row and 8 column steps
+    __shared__ double2 base[kRecAtoms][kRecGroups + 16];
+    __shared__ double fac[4][SEP ? kRecRows + kRecCols : 1];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int r0 = (wv & 1) * 16, c0 = (wv >> 1) * 32, quad = lane >> 4, l16 = lane & 15;
+    const int nrow = rec_count(p.nx, p.nmult), kc = rec_count(p.ny, p.mmult);
+    const int x0 = (int)blockIdx.y * kRecRows, y0 = (int)blockIdx.x * kRecCols - (kc - 1);  // first h and k
     const int kz = p.kz0 + (int)blockIdx.z;
-    int h, k;
-    const bool ok = refl_index(ix, p.nx, p.nmult, &h) & refl_index(iy, p.ny, p.mmult, &k);
-    const double gx = h * p.A, gy = k * p.B;
-    const double s2 = 0.25 * (gx * gx + gy * gy - 2.0 * gx * gy * p.cg);
-    // this thread's phase-factor slot: atom (tid / 32) of the chunk, column
-    // (tid % 32): 0..15 = h of tile column, 16..31 = k of tile row
-    const int slot_a = threadIdx.x >> 5, slot_c = threadIdx.x & 31;
-    int slot_q;
-    if (slot_c < 16) refl_index(blockIdx.y * 16 + slot_c, p.nx, p.nmult, &slot_q);
-    else refl_index(blockIdx.x * 16 + slot_c - 16, p.ny, p.mmult, &slot_q);
-    double vr = 0.0, vi = 0.0;
+    // sums over the species of f S and f ads S; element (t, v) of a lane is
+    // row r0 + quad + 4 v, column c0 + 16 t + l16 (the 16x16x4 FP64 layout)
+    d4 vr[2] = {}, vi[2] = {}, wr[2] = {}, wi[2] = {};
     for (int sg = p.slice_seg[kz]; sg < p.slice_seg[kz + 1]; ++sg) {
         const RecSeg seg = p.segs[sg];
-        double sr = 0.0, si = 0.0;
-        for (int a0 = seg.start; a0 < seg.end; a0 += 8) {
-            const int ai = a0 + slot_a;
-            if (ai < seg.end) {
-                const RecAtom at = p.atoms[ai];
-                double arg = (double)slot_q * (slot_c < 16 ? at.x : at.y);
-                arg -= rint(arg);
-                double sn, cs;
-                sincospi(-2.0 * arg, &sn, &cs);
-                if (slot_c < 16) {
-                    sn *= at.occ;
-                    cs *= at.occ;
-                }
-                ph[slot_a][slot_c] = make_double2(cs, sn);
-            }
+        d4 sr[2] = {}, si[2] = {};
+        if constexpr (SEP) {
+            // read after the chunks' barriers; the previous species' reads
+            // are behind the first of them
             __syncthreads();
-            const int na = min(8, seg.end - a0);
-            for (int j = 0; j < na; ++j) {
-                const double2 a = ph[j][tx], b = ph[j][16 + ty];
-                sr = fma(a.x, b.x, fma(-a.y, b.y, sr));
-                si = fma(a.x, b.y, fma(a.y, b.x, si));
-            }
-            __syncthreads();
-        }
-        double f = 0.0;
-        if (p.curves) {
-            curve_at(p.curves + (long long)seg.Z * p.npoints, p.npoints, sqrt(s2) / p.dds, &f);
-        } else {
             const double* dt = c_dt[seg.Z];
-            for (int j = 0; j < 4; ++j) f += dt[2 * j] * exp(-(dt[2 * j + 1] + seg.dw) * s2);
-            f *= p.inv_area;
+            for (int i = tid; i < 4 * (kRecRows + kRecCols); i += 256) {
+                const int j = i / (kRecRows + kRecCols), c = i % (kRecRows + kRecCols);
+                const double g = c < kRecRows ? (x0 + c) * p.A : (y0 + c - kRecRows) * p.B;
+                const double e = exp(-(dt[2 * j + 1] + seg.dw) * (0.25 * g * g));
+                fac[j][c] = c < kRecRows ? dt[2 * j] * p.inv_area * e : e;
+            }
         }
-        vr += f * (sr - seg.ads * si);
-        vi += f * (si + seg.ads * sr);
+        for (int a0 = seg.start; a0 < seg.end; a0 += kRecAtoms) {
+            for (int i = tid; i < kRecAtoms * (kRecGroups + 16); i += 256) {
+                const int j = i / (kRecGroups + 16), c = i % (kRecGroups + 16), ai = a0 + j;
+                double2 f = make_double2(0.0, 0.0);  // past the last atom: no contribution
+                if (ai < seg.end) {
+                    const RecAtom at = p.atoms[ai];
+                    const bool row = c < kRecGroups ? c < kRecRows / 8 : c < kRecGroups + 8;
+                    const int q = c >= kRecGroups ? (c - kRecGroups) & 7 : (row ? x0 + 8 * c : y0 + 8 * c - kRecRows);
+                    double arg = (double)q * (row ? at.x : at.y);
+                    arg -= rint(arg);
+                    double sn, cs;
+                    sincospi(-2.0 * arg, &sn, &cs);
+                    const double w = c < kRecRows / 8 ? at.occ : 1.0;
+                    f = make_double2(cs * w, sn * w);
+                }
+                base[j][c] = f;
+            }
+            __syncthreads();  // factors written, the previous chunk's products read
+            for (int i = tid; i < kRecAtoms * (kRecRows + kRecCols); i += 256) {
+                const int j = i / (kRecRows + kRecCols), c = i % (kRecRows + kRecCols);
+                ph[j][c] = cmul(base[j][c >> 3], base[j][kRecGroups + (c < kRecRows ? 0 : 8) + (c & 7)]);
+            }
+            __syncthreads();
+            const int na = min(kRecAtoms, seg.end - a0);
+            for (int k = 0; k < na; k += 4) {
+                const double2 a = ph[k + quad][r0 + l16];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const double2 b = ph[k + quad][kRecRows + c0 + 16 * t + l16];
+                    sr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, sr[t], 0, 0, 0);
+                    si[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.y, si[t], 0, 0, 0);
+                    sr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, b.y, sr[t], 0, 0, 0);
+                    si[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.x, si[t], 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int r = r0 + quad + 4 * v, c = c0 + 16 * t + l16;
+                double f = 0.0;
+                if constexpr (SEP) {
+                    for (int j = 0; j < 4; ++j) f += fac[j][r] * fac[j][kRecRows + c];
+                } else {
+                    const double gx = (x0 + r) * p.A, gy = (y0 + c) * p.B;
+                    const double s2 = 0.25 * (gx * gx + gy * gy - 2.0 * gx * gy * p.cg);
+                    if (p.curves) {
+                        curve_at(p.curves + (long long)seg.Z * p.npoints, p.npoints, sqrt(s2) / p.dds, &f);
+                    } else {
+                        const double* dt = c_dt[seg.Z];
+                        for (int j = 0; j < 4; ++j) f += dt[2 * j] * exp(-(dt[2 * j + 1] + seg.dw) * s2);
+                        f *= p.inv_area;
+                    }
+                }
+                vr[t][v] += f * sr[t][v];
+                vi[t][v] += f * si[t][v];
+                if constexpr (ADS) {
+                    const double fa = f * seg.ads;
+                    wr[t][v] += fa * sr[t][v];
+                    wi[t][v] += fa * si[t][v];
+                }
+            }
     }
-    if (!ok) vr = vi = 0.0;
-    p.out[((long long)blockIdx.z * p.nx + ix) * p.ny + iy] = make_double2(vr, vi);
+    double2* out = p.out + (long long)blockIdx.z * p.nx * p.ny;
+    const int half = p.nx / 2;
+    const double2 zero = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int h = x0 + r0 + quad + 4 * v, k = y0 + c0 + 16 * t + l16;
+            // column k = kc is the Nyquist column of a cell spanning the grid
+            // (otherwise a multiple beyond it, or one the clearing covers)
+            const bool ok = k < kc;
+            if (h >= nrow || k > kc || (!ok && p.mmult != 1)) continue;
+            // (1 + i ads) S, and the opposite reflection with S conjugated;
+            // row 0 is its own opposite and writes the Nyquist row's zeros
+            const double2 g = make_double2(vr[t][v] - wi[t][v], vi[t][v] + wr[t][v]);
+            const double2 m = make_double2(vr[t][v] + wi[t][v], wr[t][v] - vi[t][v]);
+            const int iy = k >= 0 ? k * p.mmult : p.ny + k * p.mmult, jy = iy == 0 ? 0 : p.ny - iy;
+            const int ix = h * p.nmult;
+            out[(long long)ix * p.ny + iy] = ok ? g : zero;
+            if (ix != 0) out[(long long)(p.nx - ix) * p.ny + jy] = ok ? m : zero;
+            else out[(long long)half * p.ny + iy] = zero;
+        }
 }
 
 hipError_t launch_rec_sf(const RecArgs& a, int nslices, hipStream_t s) {
-    dim3 grid(a.ny / 16, a.nx / 16, nslices);
-    hipLaunchKernelGGL(rec_sf_kernel, grid, dim3(256), 0, s, a);
+    const int nrow = rec_count(a.nx, a.nmult), ncol = 2 * rec_count(a.ny, a.mmult);
+    if (a.nmult != 1 || a.mmult != 1) {
+        // the indices that are no multiple keep zeros
+        hipError_t e = hipMemsetAsync(a.out, 0, sizeof(double2) * (size_t)nslices * a.nx * a.ny, s);
+        if (e != hipSuccess) return e;
+    }
+    const dim3 grid((ncol + kRecCols - 1) / kRecCols, (nrow + kRecRows - 1) / kRecRows, nslices);
+    const bool sep = std::fabs(a.cg) < 1e-15 && !a.curves;  // the cosine of a right angle given in FP64
+    if (sep && a.has_ads) hipLaunchKernelGGL((rec_sf_kernel<true, true>), grid, dim3(256), 0, s, a);
+    else if (sep) hipLaunchKernelGGL((rec_sf_kernel<false, true>), grid, dim3(256), 0, s, a);
+    else if (a.has_ads) hipLaunchKernelGGL((rec_sf_kernel<true, false>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((rec_sf_kernel<false, false>), grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
