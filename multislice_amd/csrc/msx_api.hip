@@ -210,7 +210,7 @@ struct msx_ctx_s {
     }
     std::map<int, DevBuf> tw32, tw64;
     DevBuf wave, wave2, trans, aux, tabs, partial, outbuf, atoms, cells, vtmp, curvebuf, radtab, radcoef, binbuf,
-        series;
+        series, unitbuf;
     // host side of the potential's atom binning, kept across calls (no page
     // faults on reuse); the sorted records go to pinned memory for the upload
     std::vector<long long> h_cell;
@@ -297,7 +297,7 @@ struct msx_ctx_s {
         for (auto& kv : tw64) kv.second.release();
         drop_graphs();
         for (DevBuf* b : {&wave, &wave2, &trans, &aux, &tabs, &partial, &outbuf, &atoms, &cells, &vtmp, &curvebuf, &radtab,
-                           &radcoef, &binbuf, &series})
+                           &radcoef, &binbuf, &series, &unitbuf})
             b->release();
         for (Lane& l : lanes) {
             l.wave.release();
@@ -2075,6 +2075,11 @@ int potential_rs_impl(msx_ctx ctx, const msx_atom* atoms, int64_t natoms, const 
 
 int msx_ctx_device(const msx_ctx_s* ctx) { return ctx->device; }
 hipStream_t msx_ctx_stream(const msx_ctx_s* ctx) { return ctx->stream; }
+int msx_ctx_scratch(msx_ctx_s* ctx, size_t bytes, void** out) {
+    CHK(ctx->unitbuf.ensure(bytes));
+    *out = ctx->unitbuf.p;
+    return MSX_OK;
+}
 
 // ============================================================== C ABI
 extern "C" {

@@ -27,7 +27,27 @@ struct ConvArgs {
     // partial weight gradients [splits][Cout][Cin * KS * KS], summed in a
     // fixed order into out (conv_wgrad_scratch floats; unused otherwise)
     float* partial;
+    // kFwd, kBwdData of 3x3 layers: the layer's weights packed for that mode
+    // (launch_pack_conv3), or null: the general kernel
+    const __bf16* pack;
 };
+
+// Packing of 3x3 weights into conv3's fragment order, several layers (and
+// modes) per launch.  M output rows and C reduction channels: (Cout, Cin) for
+// kFwd, (Cin, Cout) for kBwdData; offsets in elements from w and out.
+constexpr int kMaxPack = 48;
+struct PackLayer {
+    int mode, M, C;
+    long long w_off, out_off;
+};
+struct PackArgs {
+    const float* w;
+    __bf16* out;
+    PackLayer layer[kMaxPack];
+};
+size_t conv3_pack_size(int M, int C);  // elements of one layer's packed weights
+bool conv3_fits(const ConvArgs& a);    // image small enough for the packed kernel
+hipError_t launch_pack_conv3(const PackArgs& a, int layers, hipStream_t s);
 
 hipError_t launch_conv(int mode, int ks, const ConvArgs& a, hipStream_t s);
 // floats of ConvArgs::partial that launch_conv(kBwdWeight, ks, a) needs (0: none)

@@ -64,6 +64,10 @@ struct msx_unet_s {
     float* ws = nullptr;
     size_t ws_bytes = 0;
     double* partial = nullptr;
+    __bf16* pk = nullptr;   // packed 3x3 weights: every layer's kFwd, then every layer's kBwdData
+    std::vector<size_t> pk_off[2];
+    size_t pk_n[2] = {0, 0};
+    bool pk_ok[2] = {false, false};  // packed since the weights last changed
     float* wscr = nullptr;  // weight-gradient slices (conv_wgrad_scratch)
     size_t wscr_n = 0;
     std::vector<float*> ea, eb, pl, cat, da, db, g_ea, g_eb, g_pl, g_cat, g_da, g_db;
@@ -88,6 +92,7 @@ struct msx_unet_s {
         if (pbuf) hipFree(pbuf);
         if (ws) hipFree(ws);
         if (partial) hipFree(partial);
+        if (pk) hipFree(pk);
         if (wscr) hipFree(wscr);
     }
 
@@ -166,6 +171,38 @@ struct msx_unet_s {
         return MSX_OK;
     }
 
+    // offsets of the packed 3x3 weights (every layer but the head)
+    void plan_packs() {
+        for (int m = 0; m < 2; m++) {
+            pk_off[m].assign(convs.size(), 0);
+            for (size_t i = 0; i < convs.size(); i++) {
+                if (convs[i].ks != 3) continue;
+                pk_off[m][i] = pk_n[m];
+                pk_n[m] += m == kFwd ? conv3_pack_size(convs[i].cout, convs[i].cin)
+                                     : conv3_pack_size(convs[i].cin, convs[i].cout);
+            }
+        }
+    }
+    const __bf16* packed(int mode, int i) const { return pk + (mode == kFwd ? 0 : pk_n[kFwd]) + pk_off[mode][i]; }
+    // pack every 3x3 layer for `mode` if the weights have changed since
+    int pack(int mode) {
+        if (pk_ok[mode]) return MSX_OK;
+        PackArgs a{};
+        a.w = params();
+        a.out = pk + (mode == kFwd ? 0 : pk_n[kFwd]);
+        int n = 0;
+        for (size_t i = 0; i < convs.size(); i++) {
+            const ConvSpec& c = convs[i];
+            if (c.ks != 3) continue;
+            a.layer[n++] = PackLayer{mode, mode == kFwd ? c.cout : c.cin, mode == kFwd ? c.cin : c.cout,
+                                     (long long)c.w_off, (long long)pk_off[mode][i]};
+        }
+        UHIP(launch_pack_conv3(a, n, stream()));
+        pk_ok[mode] = true;
+        return MSX_OK;
+    }
+    void weights_changed() { pk_ok[kFwd] = pk_ok[kBwdData] = false; }
+
     ConvArgs conv_args(int i, int n, int l) {
         const ConvSpec& c = convs[i];
         ConvArgs a{};
@@ -184,6 +221,7 @@ struct msx_unet_s {
         a.x = x;
         a.out = y;
         a.out_c = a.Cout;
+        if (convs[i].ks == 3 && conv3_fits(a)) a.pack = packed(kFwd, i);
         UHIP(launch_conv(kFwd, convs[i].ks, a, stream()));
         return MSX_OK;
     }
@@ -212,6 +250,7 @@ struct msx_unet_s {
             a.out = gx;
             a.out_c = c.cin;
             a.accumulate = 1;
+            if (c.ks == 3 && conv3_fits(a)) a.pack = packed(kBwdData, i);
             UHIP(launch_conv(kBwdData, c.ks, a, stream()));
         }
         return MSX_OK;
@@ -220,6 +259,7 @@ struct msx_unet_s {
     // forward from xin; leaves out = xin + head(...)
     int forward() {
         const int L = levels, n = wn;
+        UCHK(pack(kFwd));
         for (int l = 0; l < L; l++) {
             UCHK(conv_fwd(enc_a(l), l, l == 0 ? xin : pl[l - 1], ea[l]));
             UCHK(conv_fwd(enc_b(l), l, ea[l], eb[l]));
@@ -242,6 +282,7 @@ struct msx_unet_s {
     int backward(double* loss) {
         const int L = levels, n = wn;
         const long long cnt = (long long)n * wh * ww;
+        UCHK(pack(kBwdData));
         // clear the accumulated gradients first: gz is the first tensor of the region
         UHIP(hipMemsetAsync(grads(), 0, nparam * sizeof(float), stream()));
         UHIP(hipMemsetAsync(grad_begin, 0, grad_bytes, stream()));
@@ -353,7 +394,9 @@ MSX_API int msx_unet_create_in(msx_ctx ctx, int levels, int base_channels, int i
         if ((int)i == net->head()) sd *= 0.1;
         for (size_t k = c.w_off; k < c.b_off; k++) p[k] = (float)(sd * nd(rng));
     }
+    net->plan_packs();
     hipError_t e = hipMalloc(&net->pbuf, 4 * off * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc(&net->pk, (net->pk_n[kFwd] + net->pk_n[kBwdData]) * sizeof(__bf16));
     if (e == hipSuccess) e = hipMalloc(&net->partial, kSqBlocks * sizeof(double));
     if (e == hipSuccess) e = hipMemcpy(net->pbuf, p.data(), off * sizeof(float), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(net->pbuf + off, 0, 3 * off * sizeof(float));
@@ -410,6 +453,16 @@ MSX_API int msx_unet_conv(msx_ctx ctx, int mode, int ks, const float* x, const f
     a.accumulate = 0;
     const size_t need = mode == kBwdWeight ? conv_wgrad_scratch(ks, a) : 0;
     if (need) UHIP(hipMalloc(&a.partial, need * sizeof(float)));
+    if (mode != kBwdWeight && ks == 3 && conv3_fits(a)) {
+        PackArgs pa{};
+        void* buf = nullptr;
+        pa.layer[0] = mode == kFwd ? PackLayer{mode, cout, cin, 0, 0} : PackLayer{mode, cin, cout, 0, 0};
+        UCHK(msx_ctx_scratch(ctx, sizeof(__bf16) * conv3_pack_size(pa.layer[0].M, pa.layer[0].C), &buf));
+        pa.w = w;
+        pa.out = static_cast<__bf16*>(buf);
+        UHIP(launch_pack_conv3(pa, 1, msx_ctx_stream(ctx)));
+        a.pack = pa.out;
+    }
     hipError_t e = launch_conv(mode, ks, a, msx_ctx_stream(ctx));
     if (e == hipSuccess) e = hipStreamSynchronize(msx_ctx_stream(ctx));
     if (a.partial) hipFree(a.partial);
@@ -437,6 +490,7 @@ MSX_API int msx_unet_set_params(msx_unet net, const float* src, int where) {
                         where == MSX_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice, net->stream()));
     UHIP(hipMemsetAsync(net->adam_m(), 0, 2 * net->nparam * sizeof(float), net->stream()));
     net->step = 0;
+    net->weights_changed();
     UHIP(hipStreamSynchronize(net->stream()));
     return MSX_OK;
 }
@@ -491,6 +545,7 @@ MSX_API int msx_unet_train_step(msx_unet net, const float* x, const float* targe
     const float c2 = (float)(1.0 - std::pow((double)b2, (double)net->step));
     UHIP(launch_adam(net->params(), net->grads(), net->adam_m(), net->adam_v(), (long long)net->nparam, lr, b1, b2,
                      eps, c1, c2, net->stream()));
+    net->weights_changed();
     UHIP(hipStreamSynchronize(net->stream()));
     return MSX_OK;
 }

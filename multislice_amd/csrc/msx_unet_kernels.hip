@@ -12,6 +12,7 @@
 // where G = dY masked by the ReLU of the layer's output.  Tensors are NCHW FP32.
 #include <hip/hip_runtime.h>
 
+#include "msx_fft.hpp"  // lds_barrier
 #include "msx_unet.h"
 
 namespace msx {
@@ -189,6 +190,184 @@ __global__ void wgrad_reduce(const float* __restrict__ part, float* out, long lo
     out[i] += s;
 }
 
+// ------------------------------------------------ 3x3 forward and input gradient
+// conv3: the products of conv_gemm's kFwd and kBwdData for 3x3 layers with the
+// operands laid out for the matrix cores.  conv_gemm gathers 8 or 16 scalars
+// per thread and 32-deep K step with one step in flight, so a step costs the
+// latency of a gather (1.8 us): a layer of 384 channels takes 108 of them.
+// Here a step is 16 input channels, 144 of K = (channel, tap): their pixels
+// with a one-pixel border are staged once in LDS (each value loaded once
+// instead of 9 times), expanded there to the 9 taps of every pixel, and feed 9
+// MFMAs per wavefront; the next step's pixels and weights load meanwhile.  The
+// weights come packed in fragment order (pack_conv3), one 16-byte load per
+// lane and MFMA.  The order of K and the position of every k in its MFMA are
+// conv_gemm's, so every output keeps its bits.
+// Bound by the latency of a step's LDS passes on small images and by LDS reads
+// (72 two-byte reads per 9 MFMAs and pixel tile) on large ones.
+//   @@@
+// Tile: PW pixel tiles of 4 x 8 pixels by 4 / PW tiles of 32 output channels,
+// one wavefront each; PW = 4 / 2 / 1 for 1 / 2-3 / more channel tiles, so that
+// a work-group's wavefronts share as much of the expansion as the layer allows.
+constexpr int kCh = 16, kK3 = kCh * 9, kSteps = kK3 / 16, kBRow = kK3 + 8;  // rows of 304 bytes: no bank conflicts
+template <int PW> struct Tile3 {
+    static constexpr int PX = PW == 4 ? 2 : 1, PY = PW / PX;   // pixel tiles along x and y
+    static constexpr int TW = 8 * PX, TH = 4 * PY, HX = TW + 2, HY = TH + 2, PS = HX * HY;
+    static constexpr int NL = (kCh * PS + 255) / 256;          // staged values per thread
+    static constexpr int G = 4 / PW;                           // groups of wavefronts that share the expansion
+};
+
+// expands runs j = G0, G0 + G, ... of 8 k: run j + 9 h holds k = 8 (j + 9 h) ..,
+// the taps of run j eight channels on, so h only moves the base address
+template <int PW, int G0> __device__ __forceinline__ void expand3(const __bf16* src, __bf16* dst) {
+    using T = Tile3<PW>;
+    bf16x8 v[(9 - G0 + T::G - 1) / T::G];
+#pragma unroll
+    for (int j = G0, i = 0; j < 9; j += T::G, ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int k = 8 * j + e, c = k / 9, t = k % 9;
+            v[i][e] = src[c * T::PS + (t / 3) * T::HX + t % 3];
+        }
+#pragma unroll
+    for (int j = G0, i = 0; j < 9; j += T::G, ++i) *reinterpret_cast<bf16x8*>(dst + 8 * j) = v[i];
+}
+
+template <int MODE, int PW> __global__ __launch_bounds__(256) void conv3(ConvArgs p) {
+    using T = Tile3<PW>;
+    __shared__ __align__(16) __bf16 Hs[T::NL * 256];
+    __shared__ __align__(16) __bf16 Bs[32 * PW][kBRow];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int M = MODE == kFwd ? p.Cout : p.Cin, C = MODE == kFwd ? p.Cin : p.Cout;
+    const int HW = p.H * p.W, nch = (C + kCh - 1) / kCh;
+    const int mt = (int)blockIdx.y * T::G + wave % T::G, pt = wave / T::G;
+    const bool mlive = mt * 32 < M;
+    const int ntx = (p.W + T::TW - 1) / T::TW, nty = (p.H + T::TH - 1) / T::TH;
+    const int img = (int)(blockIdx.x / (unsigned)(ntx * nty)), tile = (int)(blockIdx.x % (unsigned)(ntx * nty));
+    const int ty0 = tile / ntx * T::TH, tx0 = tile % ntx * T::TW;
+    // staged values: channel of the step and byte offset in its 16 planes
+    // (past the descriptor's bound outside the image: reads zero)
+    unsigned off[T::NL];
+    int ch[T::NL];
+#pragma unroll
+    for (int i = 0; i < T::NL; ++i) {
+        const int e = tid + 256 * i, q = e % T::PS;
+        ch[i] = e / T::PS;
+        const int y = ty0 + q / T::HX - 1, x = tx0 + q % T::HX - 1;
+        const bool in = (unsigned)y < (unsigned)p.H && (unsigned)x < (unsigned)p.W && ch[i] < kCh;
+        off[i] = in ? ((unsigned)ch[i] * (unsigned)HW + (unsigned)(y * p.W + x)) * 4u : 0x80000000u;
+    }
+    const float* src = (MODE == kFwd ? p.x : p.g) + (long long)img * C * HW;
+    const float* msk = MODE == kBwdData && p.relu ? p.y + (long long)img * C * HW : nullptr;
+    float v[T::NL], m[MODE == kBwdData ? T::NL : 1];
+    auto fetch = [&](int c) {
+        const int n = min(kCh, C - c * kCh);  // channels of this step; the planes past them read zero
+        const int bytes = n * HW * 4;
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(src + (long long)c * kCh * HW), 0, bytes, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < T::NL; ++i)
+            v[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int)off[i], 0, 0));
+        if constexpr (MODE == kBwdData) {
+            if (msk) {
+                const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(
+                    const_cast<float*>(msk + (long long)c * kCh * HW), 0, bytes, 0x00020000);
+#pragma unroll
+                for (int i = 0; i < T::NL; ++i)
+                    m[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rm, (int)off[i], 0, 0));
+            }
+        }
+    };
+    const __bf16* wp = p.pack + (long long)(mlive ? mt : 0) * nch * (kSteps * 512) + lane * 8;
+    bf16x8 a[kSteps], an[kSteps];
+    auto fetch_w = [&](int c, bf16x8(&w)[kSteps]) {
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s)
+            w[s] = *reinterpret_cast<const bf16x8*>(wp + ((long long)c * kSteps + s) * 512);
+    };
+    // expansion: pixel and channel half of this thread
+    const int epx = PW == 1 ? lane & 31 : (PW == 2 ? tid & 63 : tid & 127);
+    const int eh = PW == 1 ? lane >> 5 : (PW == 2 ? (tid >> 6) & 1 : tid >> 7);
+    const int eg = PW == 1 ? wave : (PW == 2 ? wave >> 1 : 0);
+    const int et = epx >> 5, el = epx & 31;
+    const __bf16* esrc = Hs + eh * 8 * T::PS + (4 * (et / T::PX) + (el >> 3)) * T::HX + 8 * (et % T::PX) + (el & 7);
+    __bf16* edst = &Bs[epx][eh * 72];
+
+    f32x16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    fetch(0);
+    fetch_w(0, a);
+    for (int c = 0; c < nch; ++c) {
+#pragma unroll
+        for (int i = 0; i < T::NL; ++i) {
+            float x = v[i];
+            if constexpr (MODE == kBwdData) {
+                if (msk && m[i] <= 0.f) x = 0.f;
+            }
+            Hs[tid + 256 * i] = (__bf16)x;
+        }
+        lds_barrier();
+        // past the last step the loads repeat it (no branch around them)
+        const int cn = min(c + 1, nch - 1);
+        fetch(cn);
+        fetch_w(cn, an);
+        if constexpr (PW == 4) expand3<PW, 0>(esrc, edst);
+        else if constexpr (PW == 2) {
+            if (eg == 0) expand3<PW, 0>(esrc, edst);
+            else expand3<PW, 1>(esrc, edst);
+        } else {
+            if (eg == 0) expand3<PW, 0>(esrc, edst);
+            else if (eg == 1) expand3<PW, 1>(esrc, edst);
+            else if (eg == 2) expand3<PW, 2>(esrc, edst);
+            else expand3<PW, 3>(esrc, edst);
+        }
+        lds_barrier();
+        const __bf16* b = &Bs[pt * 32 + (lane & 31)][(lane >> 5) * 8];
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s)
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s], *reinterpret_cast<const bf16x8*>(b + 16 * s), acc, 0, 0,
+                                                          0);
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) a[s] = an[s];
+    }
+    // acc[i] is C[row][col], col = lane % 32 (a pixel of tile pt),
+    // row = 8*(i/4) + 4*(lane/32) + i%4 (32x32 MFMA output layout)
+    const int y = ty0 + 4 * (pt / T::PX) + ((lane & 31) >> 3), x = tx0 + 8 * (pt % T::PX) + (lane & 7);
+    if (y >= p.H || x >= p.W) return;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int o = mt * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+        if (o >= M) continue;
+        float r = acc[i];
+        if (MODE == kFwd) {
+            if (p.bias) r += p.bias[o];
+            if (p.relu && r < 0.f) r = 0.f;
+        }
+        float* dst = p.out + ((long long)img * p.out_c + p.out_c0 + o) * HW + y * p.W + x;
+        if (p.accumulate) *dst += r; else *dst = r;
+    }
+}
+
+// Weights of 3x3 layers in conv3's fragment order: [tile of 32 rows m][step of
+// 16 channels][MFMA][lane][8], lane = m % 32 + 32 h holding k = 16 s + 8 h ..
+// of the step (zero past the layer's rows and channels).
+__global__ __launch_bounds__(256) void pack_conv3(PackArgs p) {
+    const PackLayer q = p.layer[blockIdx.y];
+    const int nch = (q.C + kCh - 1) / kCh;
+    const long long n = (long long)((q.M + 31) / 32) * nch * (kSteps * 512);
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
+        const int j = (int)(i & 7), lane = (int)(i >> 3) & 63;
+        const long long f = i >> 9;  // (tile, step, MFMA)
+        const int s = (int)(f % kSteps), c = (int)(f / kSteps % nch), mt = (int)(f / kSteps / nch);
+        const int m = mt * 32 + (lane & 31), k = 16 * s + 8 * (lane >> 5) + j, ch = c * kCh + k / 9, t = k % 9;
+        float w = 0.f;
+        if (m < q.M && ch < q.C)
+            w = q.mode == kFwd ? p.w[q.w_off + ((long long)m * q.C + ch) * 9 + t]
+                               : p.w[q.w_off + ((long long)ch * q.M + m) * 9 + 8 - t];
+        p.out[q.out_off + i] = (__bf16)w;
+    }
+}
+
 namespace {
 void conv_gemm_shape(int mode, int ks, const ConvArgs& a, long long* M, long long* N, long long* K) {
     const int HW = a.H * a.W;
@@ -216,12 +395,48 @@ size_t conv_wgrad_scratch(int ks, const ConvArgs& a) {
     return splits > 1 ? (size_t)splits * (size_t)(M * N) : 0;
 }
 
+size_t conv3_pack_size(int M, int C) {
+    return (size_t)((M + 31) / 32) * ((C + kCh - 1) / kCh) * (kSteps * 512);
+}
+
+hipError_t launch_pack_conv3(const PackArgs& a, int layers, hipStream_t s) {
+    hipLaunchKernelGGL(pack_conv3, dim3(64, layers), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+// conv3 takes every image whose 16 planes of a step 32-bit byte offsets reach
+// and whose tiles a grid holds; single-pixel images, a 32nd of its pixel
+// tile, stay with conv_gemm, which tiles pixels across images.
+bool conv3_fits(const ConvArgs& a) {
+    const long long hw = (long long)a.H * a.W;
+    return hw > 1 && hw <= (1 << 24) && a.N * ((a.H + 3LL) / 4) * ((a.W + 7LL) / 8) <= (1 << 21);
+}
+
+namespace {
+hipError_t launch_conv3(int mode, const ConvArgs& a, hipStream_t s) {
+    const int mt = ((mode == kFwd ? a.Cout : a.Cin) + 31) / 32, pw = mt == 1 ? 4 : (mt <= 3 ? 2 : 1);
+    const int tw = pw == 4 ? 16 : 8, th = pw == 1 ? 4 : 8, g = 4 / pw;
+    const dim3 grid((unsigned)((long long)a.N * ((a.H + th - 1) / th) * ((a.W + tw - 1) / tw)), (unsigned)((mt + g - 1) / g));
+#define MSX_CONV3(PW_)                                                                            \
+    do {                                                                                          \
+        if (mode == kFwd) hipLaunchKernelGGL((conv3<kFwd, PW_>), grid, dim3(256), 0, s, a);       \
+        else hipLaunchKernelGGL((conv3<kBwdData, PW_>), grid, dim3(256), 0, s, a);                \
+    } while (0)
+    if (pw == 4) MSX_CONV3(4);
+    else if (pw == 2) MSX_CONV3(2);
+    else MSX_CONV3(1);
+#undef MSX_CONV3
+    return hipGetLastError();
+}
+}  // namespace
+
 hipError_t launch_conv(int mode, int ks, const ConvArgs& a, hipStream_t s) {
     long long M, N, K;
     conv_gemm_shape(mode, ks, a, &M, &N, &K);
     const int bm = conv_bm(M), bn = 4096 / bm;
     const int splits = mode == kBwdWeight ? wgrad_splits(M, N, K) : 1;
     if (splits > 1 && !a.partial) return hipErrorInvalidValue;
+    if (a.pack && mode != kBwdWeight) return launch_conv3(mode, a, s);
     dim3 grid((unsigned)((N + bn - 1) / bn), (unsigned)((M + bm - 1) / bm), (unsigned)splits);
 #define MSX_CONV(MODE_, KS_, BM_) hipLaunchKernelGGL((conv_gemm<MODE_, KS_, BM_>), grid, dim3(256), 0, s, a)
 #define MSX_CONV_BM(MODE_, KS_)                    \
