@@ -198,27 +198,33 @@ __global__ void wgrad_reduce(const float* __restrict__ part, float* out, long lo
 // Here a step is 16 input channels, 144 of K = (channel, tap): their pixels
 // with a one-pixel border are staged once in LDS (each value loaded once
 // instead of 9 times), expanded there to the 9 taps of every pixel, and feed 9
-// MFMAs per wavefront; the next step's pixels and weights load meanwhile.  The
-// weights come packed in fragment order (pack_conv3), one 16-byte load per
-// lane and MFMA.  The order of K and the position of every k in its MFMA are
-// conv_gemm's, so every output keeps its bits.
-// Bound by the latency of a step's LDS passes on small images and by LDS reads
-// (72 two-byte reads per 9 MFMAs and pixel tile) on large ones.
-//   @@@
+// MFMAs per wavefront; the pixels and weights of the next two steps load
+// meanwhile.  The weights come packed in fragment order (pack_conv3), one
+// 16-byte load per lane and MFMA.  The order of K and the position of every k
+// in its MFMA are conv_gemm's, so every output keeps its bits.
+// Bound by the latency of a step's LDS passes and 9 dependent MFMAs on small
+// images (0.8 / 1.0 / 1.2 us per step for PW 1 / 2 / 4 plus 5 us per launch)
+// and by LDS reads on large ones.  The staged values are FP32: two-byte ones
+// made the compiler read pairs at odd addresses, 1.4 / 2.2 / 3.9 us per step.
+// One 128^2 image of the 4-level 32-channel network (15 layers): 826 us with
+// conv_gemm, 353 with two-byte staging and one step in flight, 249 now.
 // Tile: PW pixel tiles of 4 x 8 pixels by 4 / PW tiles of 32 output channels,
 // one wavefront each; PW = 4 / 2 / 1 for 1 / 2-3 / more channel tiles, so that
 // a work-group's wavefronts share as much of the expansion as the layer allows.
 constexpr int kCh = 16, kK3 = kCh * 9, kSteps = kK3 / 16, kBRow = kK3 + 8;  // rows of 304 bytes: no bank conflicts
 template <int PW> struct Tile3 {
     static constexpr int PX = PW == 4 ? 2 : 1, PY = PW / PX;   // pixel tiles along x and y
-    static constexpr int TW = 8 * PX, TH = 4 * PY, HX = TW + 2, HY = TH + 2, PS = HX * HY;
-    static constexpr int NL = (kCh * PS + 255) / 256;          // staged values per thread
+    static constexpr int TW = 8 * PX, TH = 4 * PY, HX = TW + 2, HY = TH + 2;
+    static constexpr int NL = (kCh * HX * HY + 255) / 256;     // staged values per thread
+    // staged rows are 24 floats apart: the 4 rows of 8 pixels that a half
+    // wavefront reads then lie in different banks
+    static constexpr int RS = 24, PS = RS * HY;
     static constexpr int G = 4 / PW;                           // groups of wavefronts that share the expansion
 };
 
 // expands runs j = G0, G0 + G, ... of 8 k: run j + 9 h holds k = 8 (j + 9 h) ..,
 // the taps of run j eight channels on, so h only moves the base address
-template <int PW, int G0> __device__ __forceinline__ void expand3(const __bf16* src, __bf16* dst) {
+template <int PW, int G0> __device__ __forceinline__ void expand3(const float* src, __bf16* dst) {
     using T = Tile3<PW>;
     bf16x8 v[(9 - G0 + T::G - 1) / T::G];
 #pragma unroll
@@ -226,7 +232,7 @@ template <int PW, int G0> __device__ __forceinline__ void expand3(const __bf16* 
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int k = 8 * j + e, c = k / 9, t = k % 9;
-            v[i][e] = src[c * T::PS + (t / 3) * T::HX + t % 3];
+            v[i][e] = (__bf16)src[c * T::PS + (t / 3) * T::RS + t % 3];
         }
 #pragma unroll
     for (int j = G0, i = 0; j < 9; j += T::G, ++i) *reinterpret_cast<bf16x8*>(dst + 8 * j) = v[i];
@@ -234,7 +240,7 @@ template <int PW, int G0> __device__ __forceinline__ void expand3(const __bf16* 
 
 template <int MODE, int PW> __global__ __launch_bounds__(256) void conv3(ConvArgs p) {
     using T = Tile3<PW>;
-    __shared__ __align__(16) __bf16 Hs[T::NL * 256];
+    __shared__ float Hs[kCh * T::PS];
     __shared__ __align__(16) __bf16 Bs[32 * PW][kBRow];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int M = MODE == kFwd ? p.Cout : p.Cin, C = MODE == kFwd ? p.Cin : p.Cout;
@@ -244,22 +250,25 @@ template <int MODE, int PW> __global__ __launch_bounds__(256) void conv3(ConvArg
     const int ntx = (p.W + T::TW - 1) / T::TW, nty = (p.H + T::TH - 1) / T::TH;
     const int img = (int)(blockIdx.x / (unsigned)(ntx * nty)), tile = (int)(blockIdx.x % (unsigned)(ntx * nty));
     const int ty0 = tile / ntx * T::TH, tx0 = tile % ntx * T::TW;
-    // staged values: channel of the step and byte offset in its 16 planes
-    // (past the descriptor's bound outside the image: reads zero)
+    // staged values: byte offset in the step's 16 planes (past the
+    // descriptor's bound outside the image: reads zero) and place in Hs
     unsigned off[T::NL];
-    int ch[T::NL];
+    int pos[T::NL];
 #pragma unroll
     for (int i = 0; i < T::NL; ++i) {
-        const int e = tid + 256 * i, q = e % T::PS;
-        ch[i] = e / T::PS;
+        const int e = tid + 256 * i, ch = e / (T::HX * T::HY), q = e % (T::HX * T::HY);
         const int y = ty0 + q / T::HX - 1, x = tx0 + q % T::HX - 1;
-        const bool in = (unsigned)y < (unsigned)p.H && (unsigned)x < (unsigned)p.W && ch[i] < kCh;
-        off[i] = in ? ((unsigned)ch[i] * (unsigned)HW + (unsigned)(y * p.W + x)) * 4u : 0x80000000u;
+        const bool in = (unsigned)y < (unsigned)p.H && (unsigned)x < (unsigned)p.W && ch < kCh;
+        off[i] = in ? ((unsigned)ch * (unsigned)HW + (unsigned)(y * p.W + x)) * 4u : 0x80000000u;
+        // what is left over past the last channel goes to a pad of the last row
+        pos[i] = ch < kCh ? ch * T::PS + (q / T::HX) * T::RS + q % T::HX : kCh * T::PS - 1;
     }
     const float* src = (MODE == kFwd ? p.x : p.g) + (long long)img * C * HW;
     const float* msk = MODE == kBwdData && p.relu ? p.y + (long long)img * C * HW : nullptr;
-    float v[T::NL], m[MODE == kBwdData ? T::NL : 1];
-    auto fetch = [&](int c) {
+    constexpr int NM = MODE == kBwdData ? T::NL : 1;
+    // past the last step the loads repeat it (no branch around them)
+    auto fetch = [&](int c, float(&v)[T::NL], float(&m)[NM]) {
+        c = min(c, nch - 1);
         const int n = min(kCh, C - c * kCh);  // channels of this step; the planes past them read zero
         const int bytes = n * HW * 4;
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
@@ -278,8 +287,8 @@ template <int MODE, int PW> __global__ __launch_bounds__(256) void conv3(ConvArg
         }
     };
     const __bf16* wp = p.pack + (long long)(mlive ? mt : 0) * nch * (kSteps * 512) + lane * 8;
-    bf16x8 a[kSteps], an[kSteps];
     auto fetch_w = [&](int c, bf16x8(&w)[kSteps]) {
+        c = min(c, nch - 1);
 #pragma unroll
         for (int s = 0; s < kSteps; ++s)
             w[s] = *reinterpret_cast<const bf16x8*>(wp + ((long long)c * kSteps + s) * 512);
@@ -289,28 +298,26 @@ template <int MODE, int PW> __global__ __launch_bounds__(256) void conv3(ConvArg
     const int eh = PW == 1 ? lane >> 5 : (PW == 2 ? (tid >> 6) & 1 : tid >> 7);
     const int eg = PW == 1 ? wave : (PW == 2 ? wave >> 1 : 0);
     const int et = epx >> 5, el = epx & 31;
-    const __bf16* esrc = Hs + eh * 8 * T::PS + (4 * (et / T::PX) + (el >> 3)) * T::HX + 8 * (et % T::PX) + (el & 7);
+    const float* esrc = Hs + eh * 8 * T::PS + (4 * (et / T::PX) + (el >> 3)) * T::RS + 8 * (et % T::PX) + (el & 7);
     __bf16* edst = &Bs[epx][eh * 72];
 
     f32x16 acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-    fetch(0);
-    fetch_w(0, a);
-    for (int c = 0; c < nch; ++c) {
+    // one step: its pixels are in v (mask source in m), its weights in w; once
+    // consumed, the registers take those of the step after next
+    auto step = [&](int c, float(&v)[T::NL], float(&m)[NM], bf16x8(&w)[kSteps]) {
 #pragma unroll
         for (int i = 0; i < T::NL; ++i) {
             float x = v[i];
             if constexpr (MODE == kBwdData) {
                 if (msk && m[i] <= 0.f) x = 0.f;
             }
-            Hs[tid + 256 * i] = (__bf16)x;
+            Hs[pos[i]] = x;
         }
+        fetch(c + 2, v, m);
+        __builtin_amdgcn_sched_barrier(0);
         lds_barrier();
-        // past the last step the loads repeat it (no branch around them)
-        const int cn = min(c + 1, nch - 1);
-        fetch(cn);
-        fetch_w(cn, an);
         if constexpr (PW == 4) expand3<PW, 0>(esrc, edst);
         else if constexpr (PW == 2) {
             if (eg == 0) expand3<PW, 0>(esrc, edst);
@@ -325,26 +332,48 @@ template <int MODE, int PW> __global__ __launch_bounds__(256) void conv3(ConvArg
         const __bf16* b = &Bs[pt * 32 + (lane & 31)][(lane >> 5) * 8];
 #pragma unroll
         for (int s = 0; s < kSteps; ++s)
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s], *reinterpret_cast<const bf16x8*>(b + 16 * s), acc, 0, 0,
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[s], *reinterpret_cast<const bf16x8*>(b + 16 * s), acc, 0, 0,
                                                           0);
-#pragma unroll
-        for (int s = 0; s < kSteps; ++s) a[s] = an[s];
+        fetch_w(c + 2, w);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    float v0[T::NL], v1[T::NL], m0[NM], m1[NM];
+    bf16x8 w0[kSteps], w1[kSteps];
+    // in the loop's issue order: the wait counters count in order, and a value
+    // loaded later here than there makes the loop wait for everything
+    fetch(0, v0, m0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_w(0, w0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(1, v1, m1);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_w(1, w1);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int c = 0; c < nch; c += 2) {
+        step(c, v0, m0, w0);
+        if (c + 1 < nch) step(c + 1, v1, m1, w1);
     }
     // acc[i] is C[row][col], col = lane % 32 (a pixel of tile pt),
-    // row = 8*(i/4) + 4*(lane/32) + i%4 (32x32 MFMA output layout)
+    // row = 8*(i/4) + 4*(lane/32) + i%4 (32x32 MFMA output layout).  What the
+    // outputs need is loaded before the first store, dead rows from a valid
+    // address: one wait instead of one per output
     const int y = ty0 + 4 * (pt / T::PX) + ((lane & 31) >> 3), x = tx0 + 8 * (pt % T::PX) + (lane & 7);
     if (y >= p.H || x >= p.W) return;
+    float* const out0 = p.out + ((long long)img * p.out_c + p.out_c0) * HW + y * p.W + x;
+    const int o0 = mt * 32 + 4 * (lane >> 5);
+    float add[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        const int o = mt * 32 + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-        if (o >= M) continue;
-        float r = acc[i];
-        if (MODE == kFwd) {
-            if (p.bias) r += p.bias[o];
-            if (p.relu && r < 0.f) r = 0.f;
-        }
-        float* dst = p.out + ((long long)img * p.out_c + p.out_c0 + o) * HW + y * p.W + x;
-        if (p.accumulate) *dst += r; else *dst = r;
+        const int o = o0 + 8 * (i >> 2) + (i & 3);
+        if (MODE == kFwd) add[i] = p.bias ? p.bias[min(o, M - 1)] : 0.f;
+        else add[i] = p.accumulate ? out0[(long long)min(o, M - 1) * HW] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int o = o0 + 8 * (i >> 2) + (i & 3);
+        float r = acc[i] + add[i];
+        if (MODE == kFwd && p.relu && r < 0.f) r = 0.f;
+        if (o < M) out0[(long long)o * HW] = r;
     }
 }
 
