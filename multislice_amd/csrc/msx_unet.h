@@ -30,6 +30,16 @@ struct ConvArgs {
     // kFwd, kBwdData of 3x3 layers: the layer's weights packed for that mode
     // (launch_pack_conv3), or null: the general kernel
     const __bf16* pack;
+    // kFwd with pack: further copies of the output, each optional: its 2x2
+    // average [N, Cout, H/2, W/2] (H, W even), itself as channels skip_c0 ..
+    // of a tensor with skip_c channels, and its nearest x2 upsampling as the
+    // first channels of a [N, up_c, 2H, 2W] tensor
+    float *pool, *skip, *up;
+    int skip_c, skip_c0, up_c;
+    // kFwd without pack: out = mean over res_c channels of res [N, res_c, H, W]
+    // + the convolution (one output channel), or null
+    const float* res;
+    int res_c;
 };
 
 // Packing of 3x3 weights into conv3's fragment order, several layers (and

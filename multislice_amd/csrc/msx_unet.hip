@@ -72,7 +72,7 @@ struct msx_unet_s {
     size_t wscr_n = 0;
     std::vector<float*> ea, eb, pl, cat, da, db, g_ea, g_eb, g_pl, g_cat, g_da, g_db;
     float *xin = nullptr, *tin = nullptr, *z = nullptr, *out = nullptr, *gz = nullptr;
-    float* xbase = nullptr;  // channel mean of xin (xin itself with one channel)
+    float* xbase = nullptr;  // channel mean of the inputs (with more than one channel)
     float* grad_begin = nullptr;
     size_t grad_bytes = 0;
 
@@ -162,7 +162,6 @@ struct msx_unet_s {
             ws_bytes = bytes;
         }
         for (size_t i = 0; i < slots.size(); i++) *slots[i].dst = ws + offs[i];
-        if (cin0 == 1) xbase = xin;
         grad_begin = ws + offs[grad_first];
         grad_bytes = (total - offs[grad_first]) * sizeof(float);
         wn = n;
@@ -216,12 +215,26 @@ struct msx_unet_s {
         a.relu = c.relu;
         return a;
     }
-    int conv_fwd(int i, int l, const float* x, float* y) {
+    // does layer i at level l run the packed kernel?
+    bool packs(int i, int l) { return convs[i].ks == 3 && conv3_fits(conv_args(i, wn, l)); }
+    // a: the extra outputs (pool, skip, up) of the packed kernel or the
+    // residual of the head
+    int conv_fwd(int i, int l, const float* x, float* y, const ConvArgs* extra = nullptr) {
         ConvArgs a = conv_args(i, wn, l);
+        if (extra) {
+            a.pool = extra->pool;
+            a.skip = extra->skip;
+            a.skip_c = extra->skip_c;
+            a.skip_c0 = extra->skip_c0;
+            a.up = extra->up;
+            a.up_c = extra->up_c;
+            a.res = extra->res;
+            a.res_c = extra->res_c;
+        }
         a.x = x;
         a.out = y;
         a.out_c = a.Cout;
-        if (convs[i].ks == 3 && conv3_fits(a)) a.pack = packed(kFwd, i);
+        if (packs(i, l)) a.pack = packed(kFwd, i);
         UHIP(launch_conv(kFwd, convs[i].ks, a, stream()));
         return MSX_OK;
     }
@@ -250,44 +263,71 @@ struct msx_unet_s {
             a.out = gx;
             a.out_c = c.cin;
             a.accumulate = 1;
-            if (c.ks == 3 && conv3_fits(a)) a.pack = packed(kBwdData, i);
+            if (packs(i, l)) a.pack = packed(kBwdData, i);
             UHIP(launch_conv(kBwdData, c.ks, a, stream()));
         }
         return MSX_OK;
     }
 
-    // forward from xin; leaves out = xin + head(...)
-    int forward() {
+    // forward from x; leaves the head's output in z, or with y set writes
+    // mean(x) + head there.  The packed kernel writes the pooled, skipped and
+    // upsampled copies of its outputs itself (each was a launch of 4-5 us).
+    int forward(const float* x, float* y = nullptr) {
         const int L = levels, n = wn;
         UCHK(pack(kFwd));
         for (int l = 0; l < L; l++) {
-            UCHK(conv_fwd(enc_a(l), l, l == 0 ? xin : pl[l - 1], ea[l]));
-            UCHK(conv_fwd(enc_b(l), l, ea[l], eb[l]));
-            if (l < L - 1) UHIP(launch_avgpool_fwd(eb[l], pl[l], (long long)n * C(l), wh >> l, ww >> l, stream()));
+            UCHK(conv_fwd(enc_a(l), l, l == 0 ? x : pl[l - 1], ea[l]));
+            ConvArgs e{};
+            const bool fused = packs(enc_b(l), l);
+            if (fused && l < L - 1) {
+                e.pool = pl[l];
+                e.skip = cat[l];
+                e.skip_c = C(l + 1) + C(l);
+                e.skip_c0 = C(l + 1);
+            } else if (fused && L > 1) {
+                e.up = cat[l - 1];
+                e.up_c = C(l) + C(l - 1);
+            }
+            UCHK(conv_fwd(enc_b(l), l, ea[l], eb[l], &e));
+            if (!fused && l < L - 1) {
+                UHIP(launch_avgpool_fwd(eb[l], pl[l], (long long)n * C(l), wh >> l, ww >> l, stream()));
+                UHIP(launch_copy_channels(eb[l], C(l), 0, cat[l], C(l + 1) + C(l), C(l + 1), n, C(l),
+                                          (wh >> l) * (ww >> l), 0, stream()));
+            }
         }
         const float* prev = eb[L - 1];
         for (int l = L - 2; l >= 0; l--) {
             const int Ct = C(l + 1) + C(l), hl = wh >> l, wl = ww >> l;
-            UHIP(launch_upsample_fwd(prev, cat[l], n, C(l + 1), hl / 2, wl / 2, Ct, 0, stream()));
-            UHIP(launch_copy_channels(eb[l], C(l), 0, cat[l], Ct, C(l + 1), n, C(l), hl * wl, 0, stream()));
+            if (!packs(l + 1 == L - 1 ? enc_b(l + 1) : dec_b(l + 1), l + 1))
+                UHIP(launch_upsample_fwd(prev, cat[l], n, C(l + 1), hl / 2, wl / 2, Ct, 0, stream()));
             UCHK(conv_fwd(dec_a(l), l, cat[l], da[l]));
-            UCHK(conv_fwd(dec_b(l), l, da[l], db[l]));
+            ConvArgs e{};
+            if (l > 0 && packs(dec_b(l), l)) {
+                e.up = cat[l - 1];
+                e.up_c = C(l) + C(l - 1);
+            }
+            UCHK(conv_fwd(dec_b(l), l, da[l], db[l], &e));
             prev = db[l];
         }
-        UCHK(conv_fwd(head(), 0, prev, z));
+        ConvArgs e{};
+        if (y) {
+            e.res = x;
+            e.res_c = cin0;
+        }
+        UCHK(conv_fwd(head(), 0, prev, y ? y : z, &e));
         return MSX_OK;
     }
 
     // loss = mean (out - t)^2 (out computed here), and every gradient
-    int backward(double* loss) {
+    int backward(const float* x, const float* t, double* loss) {
         const int L = levels, n = wn;
         const long long cnt = (long long)n * wh * ww;
         UCHK(pack(kBwdData));
         // clear the accumulated gradients first: gz is the first tensor of the region
         UHIP(hipMemsetAsync(grads(), 0, nparam * sizeof(float), stream()));
         UHIP(hipMemsetAsync(grad_begin, 0, grad_bytes, stream()));
-        UHIP(launch_residual_mse(xbase, z, tin, out, gz, cnt, 2.0f / (float)cnt, stream()));
-        UHIP(launch_sq_diff(out, tin, cnt, partial, kSqBlocks, stream()));
+        UHIP(launch_residual_mse(cin0 > 1 ? xbase : x, z, t, out, gz, cnt, 2.0f / (float)cnt, stream()));
+        UHIP(launch_sq_diff(out, t, cnt, partial, kSqBlocks, stream()));
         const float* prev = L > 1 ? db[0] : eb[0];
         float* g_prev = L > 1 ? g_db[0] : g_eb[0];
         UCHK(conv_bwd(head(), 0, prev, z, gz, g_prev));
@@ -301,7 +341,7 @@ struct msx_unet_s {
         }
         for (int l = L - 1; l >= 0; l--) {
             UCHK(conv_bwd(enc_b(l), l, ea[l], eb[l], g_eb[l], g_ea[l]));
-            UCHK(conv_bwd(enc_a(l), l, l == 0 ? xin : pl[l - 1], ea[l], g_ea[l], l > 0 ? g_pl[l - 1] : nullptr));
+            UCHK(conv_bwd(enc_a(l), l, l == 0 ? x : pl[l - 1], ea[l], g_ea[l], l > 0 ? g_pl[l - 1] : nullptr));
             if (l > 0)
                 UHIP(launch_avgpool_bwd(g_pl[l - 1], g_eb[l - 1], (long long)n * C(l - 1), wh >> (l - 1),
                                         ww >> (l - 1), stream()));
@@ -333,16 +373,24 @@ int check_shape(msx_unet net, int n, int h, int w, int where) {
     if ((long long)n * h * w > (1LL << 26)) return fail(MSX_EINVAL, "batch of %lld pixels too large", (long long)n * h * w);
     return MSX_OK;
 }
-// stage the inputs (x [n][cin0][h][w], optional target [n][h][w]) into the
-// workspace, with the channel mean of x for the residual
-int stage_inputs(msx_unet net, const float* x, const float* t, int where) {
-    const size_t npix = (size_t)net->wn * net->wh * net->ww, bytes = sizeof(float) * npix;
-    const hipMemcpyKind k = where == MSX_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
-    UHIP(hipMemcpyAsync(net->xin, x, bytes * net->cin0, k, net->stream()));
+// the inputs (*x [n][cin0][h][w], optional target *t [n][h][w]) on the GPU:
+// device tensors are read where they are (every call waits for its work),
+// host ones are copied into the workspace
+int stage_inputs(msx_unet net, const float** x, const float** t, int where) {
+    if (where == MSX_DEVICE) return MSX_OK;
+    const size_t bytes = sizeof(float) * (size_t)net->wn * net->wh * net->ww;
+    UHIP(hipMemcpyAsync(net->xin, *x, bytes * net->cin0, hipMemcpyHostToDevice, net->stream()));
+    *x = net->xin;
+    if (t) {
+        UHIP(hipMemcpyAsync(net->tin, *t, bytes, hipMemcpyHostToDevice, net->stream()));
+        *t = net->tin;
+    }
+    return MSX_OK;
+}
+// channel mean of the staged inputs, for the residual of a training step
+int stage_mean(msx_unet net, const float* x) {
     if (net->cin0 > 1)
-        UHIP(launch_channel_mean(net->xin, net->xbase, net->wn, net->cin0, (long long)net->wh * net->ww,
-                                 net->stream()));
-    if (t) UHIP(hipMemcpyAsync(net->tin, t, bytes, k, net->stream()));
+        UHIP(launch_channel_mean(x, net->xbase, net->wn, net->cin0, (long long)net->wh * net->ww, net->stream()));
     return MSX_OK;
 }
 
@@ -501,12 +549,16 @@ MSX_API int msx_unet_forward(msx_unet net, const float* x, float* y, int n, int 
     if (!x || !y) return fail(MSX_EINVAL, "x and y must be non-NULL");
     UHIP(hipSetDevice(msx_ctx_device(net->ctx)));
     UCHK(net->workspace(n, h, w));
-    UCHK(stage_inputs(net, x, nullptr, where));
-    UCHK(net->forward());
-    const long long cnt = (long long)n * h * w;
-    UHIP(launch_residual_mse(net->xbase, net->z, nullptr, net->out, nullptr, cnt, 0.f, net->stream()));
-    UHIP(hipMemcpyAsync(y, net->out, sizeof(float) * cnt,
-                        where == MSX_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice, net->stream()));
+    UCHK(stage_inputs(net, &x, nullptr, where));
+    // straight into y unless it is a host buffer or shares memory with x
+    // (the head's tiles read x while others write)
+    const size_t cnt = (size_t)n * h * w;
+    const bool apart = y + cnt <= x || x + cnt * net->cin0 <= y;
+    float* dst = where == MSX_DEVICE && apart ? y : net->out;
+    UCHK(net->forward(x, dst));
+    if (dst != y)
+        UHIP(hipMemcpyAsync(y, dst, sizeof(float) * cnt,
+                            where == MSX_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice, net->stream()));
     UHIP(hipStreamSynchronize(net->stream()));
     return MSX_OK;
 }
@@ -518,9 +570,10 @@ MSX_API int msx_unet_gradient(msx_unet net, const float* x, const float* target,
     if (!x || !target) return fail(MSX_EINVAL, "x and target must be non-NULL");
     UHIP(hipSetDevice(msx_ctx_device(net->ctx)));
     UCHK(net->workspace(n, h, w));
-    UCHK(stage_inputs(net, x, target, where));
-    UCHK(net->forward());
-    UCHK(net->backward(loss));
+    UCHK(stage_inputs(net, &x, &target, where));
+    UCHK(stage_mean(net, x));
+    UCHK(net->forward(x));
+    UCHK(net->backward(x, target, loss));
     if (grad)
         UHIP(hipMemcpyAsync(grad, net->grads(), net->nparam * sizeof(float),
                             where == MSX_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice, net->stream()));
@@ -536,9 +589,10 @@ MSX_API int msx_unet_train_step(msx_unet net, const float* x, const float* targe
     if (!(lr > 0.f)) return fail(MSX_EINVAL, "lr must be > 0");
     UHIP(hipSetDevice(msx_ctx_device(net->ctx)));
     UCHK(net->workspace(n, h, w));
-    UCHK(stage_inputs(net, x, target, where));
-    UCHK(net->forward());
-    UCHK(net->backward(loss));
+    UCHK(stage_inputs(net, &x, &target, where));
+    UCHK(stage_mean(net, x));
+    UCHK(net->forward(x));
+    UCHK(net->backward(x, target, loss));
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     net->step++;
     const float c1 = (float)(1.0 - std::pow((double)b1, (double)net->step));

@@ -171,6 +171,17 @@ __global__ __launch_bounds__(256) void conv_gemm(ConvArgs p) {
         if (MODE == kFwd || MODE == kBwdData) {
             const int img = (int)(n / HW), pix = (int)(n % HW);
             float* dst = p.out + ((long long)img * p.out_c + p.out_c0 + m) * HW + pix;
+            if (MODE == kFwd && p.res) {
+                // the mean as launch_channel_mean forms it
+                const float* q = p.res + (long long)img * p.res_c * HW + pix;
+                float b = q[0];
+                if (p.res_c > 1) {
+                    b = 0.f;
+                    for (int k = 0; k < p.res_c; ++k) b += q[(long long)k * HW];
+                    b = b * (1.0f / (float)p.res_c);
+                }
+                c = b + c;
+            }
             if (p.accumulate) *dst += c; else *dst = c;
         } else if (gridDim.z > 1) {
             // this reduction slice's share of dW[co][ci][tap]; wgrad_reduce
@@ -207,7 +218,9 @@ __global__ void wgrad_reduce(const float* __restrict__ part, float* out, long lo
 // and by LDS reads on large ones.  The staged values are FP32: two-byte ones
 // made the compiler read pairs at odd addresses, 1.4 / 2.2 / 3.9 us per step.
 // One 128^2 image of the 4-level 32-channel network (15 layers): 826 us with
-// conv_gemm, 353 with two-byte staging and one step in flight, 249 now.
+// conv_gemm, 353 with two-byte staging and one step in flight, 249 with FP32
+// staging and two; 219 with the pooled, concatenated and upsampled copies and
+// the residual written by the epilogues instead of 12 launches and 2 copies.
 // Tile: PW pixel tiles of 4 x 8 pixels by 4 / PW tiles of 32 output channels,
 // one wavefront each; PW = 4 / 2 / 1 for 1 / 2-3 / more channel tiles, so that
 // a work-group's wavefronts share as much of the expansion as the layer allows.
@@ -358,7 +371,7 @@ template <int MODE, int PW> __global__ __launch_bounds__(256) void conv3(ConvArg
     // outputs need is loaded before the first store, dead rows from a valid
     // address: one wait instead of one per output
     const int y = ty0 + 4 * (pt / T::PX) + ((lane & 31) >> 3), x = tx0 + 8 * (pt % T::PX) + (lane & 7);
-    if (y >= p.H || x >= p.W) return;
+    if (y >= p.H || x >= p.W) return;  // whole 2x2 groups (an even image) or none of one
     float* const out0 = p.out + ((long long)img * p.out_c + p.out_c0) * HW + y * p.W + x;
     const int o0 = mt * 32 + 4 * (lane >> 5);
     float add[16];
@@ -373,6 +386,24 @@ template <int MODE, int PW> __global__ __launch_bounds__(256) void conv3(ConvArg
         const int o = o0 + 8 * (i >> 2) + (i & 3);
         float r = acc[i] + add[i];
         if (MODE == kFwd && p.relu && r < 0.f) r = 0.f;
+        if constexpr (MODE == kFwd) {
+            if (p.pool) {
+                // the 2x2 group's values are in this lane and the lanes one
+                // and eight up (8 pixels per row); lane bits 0 and 3 clear hold
+                // its first pixel.  H and W are even: the group is whole
+                const float s1 = __shfl_down(r, 1, 64), s2 = __shfl_down(r, 8, 64), s3 = __shfl_down(r, 9, 64);
+                if (o < M && (lane & 9) == 0)
+                    p.pool[((long long)img * M + o) * (HW >> 2) + (y >> 1) * (p.W >> 1) + (x >> 1)] =
+                        0.25f * (r + s1 + s2 + s3);
+            }
+            if (p.skip && o < M) p.skip[((long long)img * p.skip_c + p.skip_c0 + o) * HW + y * p.W + x] = r;
+            if (p.up && o < M) {
+                float* u = p.up + ((long long)img * p.up_c + o) * (4ll * HW) + (long long)(4 * y) * p.W + 2 * x;
+                const float2 rr = make_float2(r, r);
+                *reinterpret_cast<float2*>(u) = rr;
+                *reinterpret_cast<float2*>(u + 2 * p.W) = rr;
+            }
+        }
         if (o < M) out0[(long long)o * HW] = r;
     }
 }
