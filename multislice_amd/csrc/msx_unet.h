@@ -27,6 +27,7 @@ struct ConvArgs {
     // partial weight gradients [splits][Cout][Cin * KS * KS], summed in a
     // fixed order into out (conv_wgrad_scratch floats; unused otherwise)
     float* partial;
+    float* db;  // kBwdWeight: bias gradient [Cout], or null
     // kFwd, kBwdData of 3x3 layers: the layer's weights packed for that mode
     // (launch_pack_conv3), or null: the general kernel
     const __bf16* pack;
@@ -68,7 +69,6 @@ hipError_t launch_upsample_fwd(const float* x, float* y, int N, int C, int H, in
 hipError_t launch_upsample_bwd(const float* gy, float* gx, int N, int C, int H, int W, int Ct, int c0, hipStream_t s);
 hipError_t launch_copy_channels(const float* src, int Cs, int s0, float* dst, int Cd, int d0, int N, int C, int HW,
                                 int accumulate, hipStream_t s);
-hipError_t launch_bias_grad(const float* g, const float* y, int relu, int N, int C, int HW, float* db, hipStream_t s);
 hipError_t launch_residual_mse(const float* in, const float* z, const float* t, float* out, float* g, long long n,
                                float scale, hipStream_t s);
 // y[n][p] = (1/C) sum_c x[n][c][p] (FP32, channels in order)

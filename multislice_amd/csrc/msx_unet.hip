@@ -257,8 +257,8 @@ struct msx_unet_s {
             wscr_n = need;
         }
         a.partial = wscr;
+        a.db = grads() + c.b_off;
         UHIP(launch_conv(kBwdWeight, c.ks, a, stream()));
-        UHIP(launch_bias_grad(g, y, c.relu, wn, c.cout, a.H * a.W, grads() + c.b_off, stream()));
         if (gx) {
             a.out = gx;
             a.out_c = c.cin;
