@@ -131,6 +131,17 @@ int fidx(int i, int n) {
     int imid = (int)(n / 2.0 + 0.5);
     return i > imid ? i - n : i;
 }
+// The y columns in band (ky2 < k2max): iy < lo and iy >= ny - hi (ky2 rises
+// with |ky| on both sides of 0).
+struct Band {
+    int lo = 0, hi = 0;
+};
+Band band_limits(const float* ky2_host, int ny, float k2max) {
+    Band b;
+    while (b.lo < ny && ky2_host[b.lo] < k2max) b.lo++;
+    while (b.hi < ny - b.lo && ky2_host[ny - 1 - b.hi] < k2max) b.hi++;
+    return b;
+}
 // fraction of y columns inside the band (host copy of the kernels' test)
 double band_fraction(const float* ky2_host, int ny, float k2max) {
     int k = 0;
@@ -336,6 +347,7 @@ template <typename C> struct SliceTables {
     const C* px = nullptr;  // [nlayer][nx]
     const C* py = nullptr;  // [nlayer][ny]
     float k2max = 0.f;
+    Band band;  // the y columns with ky2 < k2max
     // twiddles of the x and y transforms; null: the context's cached tables
     const C* twx = nullptr;
     const C* twy = nullptr;
@@ -403,6 +415,7 @@ int upload_tables(msx_ctx ctx, const msx_stack* st, const HostTables<C>& h, char
     out->px = reinterpret_cast<const C*>(base + h.o_px);
     out->py = reinterpret_cast<const C*>(base + h.o_py);
     out->k2max = k2max_of(nx, ny, st->ax, st->by, st->bw);
+    out->band = band_limits(h.ky2.data(), ny, out->k2max);
     ctx->band = band_fraction(h.ky2.data(), ny, out->k2max);
     return MSX_OK;
 }
@@ -518,21 +531,20 @@ int transmission_dev(msx_ctx ctx, const typename real_of<C>::type* V, int nl, in
     // column with ky2 >= k2max, so the forward row sweep does not store
     // those columns, the column sweep skips them, and the inverse row sweep
     // takes them as zeros without loading them (and stores the full image).
-    r.ky2 = tb.ky2;
-    r.k2max = tb.k2max;
+    r.blo = tb.band.lo, r.bhi = tb.band.hi;
     r.prune = 2;
     LAUNCH_ROW(ny, kRowFwd, r);
     ColArgs<C> c = col_args<C>(t, ny, nl, twx);
     c.kx2 = tb.kx2;
     c.ky2 = tb.ky2;
     c.k2max = tb.k2max;
+    c.blo = tb.band.lo, c.bhi = tb.band.hi;
     c.prune = 1;
     c.ops = kColMask | kColStore;
     LAUNCH_COL(nx, kColSlice, c);
     RowArgs<C> r2 = row_args<C>(t, nx, nl, twy);
     r2.scale = (Re)1 / ((Re)nx * (Re)ny);
-    r2.ky2 = tb.ky2;
-    r2.k2max = tb.k2max;
+    r2.blo = tb.band.lo, r2.bhi = tb.band.hi;
     r2.prune = 1;
     LAUNCH_ROW(ny, kRowInv, r2);
     return MSX_OK;
@@ -589,8 +601,7 @@ int series_records(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, C
         r.src = psi;
         r.src_bstride = img;
         r.scale = (Re)1 / ((Re)nx * (Re)ny);
-        r.ky2 = tb.ky2;
-        r.k2max = tb.k2max;
+        r.blo = tb.band.lo, r.bhi = tb.band.hi;
         r.prune = obl ? 0 : 1;
         LAUNCH_ROW(ny, kRowInv, r);
         ser->iat++;
@@ -635,8 +646,7 @@ int slice_loop_body(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, 
         // (prune & 2: the next column sweep skips them).
         RowArgs<C> r = row_args<C>(psi, nx, nb, twy);
         r.trans = trans + (long long)l * img;
-        r.ky2 = tb.ky2;
-        r.k2max = tb.k2max;
+        r.blo = tb.band.lo, r.bhi = tb.band.hi;
         r.prune = obl ? 0 : ((s == 0) ? 2 : 3);
         if (tu) r.wpb = tu->row_wpb, r.plan = tu->row_plan;
         if (s == 0 && start == 0) {
@@ -652,6 +662,7 @@ int slice_loop_body(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, 
         c.kx2 = tb.kx2;
         c.ky2 = tb.ky2;
         c.k2max = tb.k2max;
+        c.blo = tb.band.lo, c.bhi = tb.band.hi;
         c.px = tb.px + (long long)l * nx;
         c.py = tb.py + (long long)l * ny;
         c.ops = kColProp | kColStore;
@@ -707,8 +718,7 @@ int slice_loop_body(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, 
     if (!det && !mixed_out) {
         RowArgs<C> r = row_args<C>(psi, nx, nb, twy);
         r.scale = inv;
-        r.ky2 = tb.ky2;
-        r.k2max = tb.k2max;
+        r.blo = tb.band.lo, r.bhi = tb.band.hi;
         r.prune = obl ? 0 : 1;
         if (tu) r.plan = tu->row_plan;
         LAUNCH_ROW(ny, kRowInv, r);
@@ -1013,8 +1023,7 @@ int batch_class(msx_ctx ctx, const msx_job* jobs, std::vector<BatchItem>& g, std
         const int na = active[s];
         RowArgs<C> r = row_args<C>(w, nx, na, twy);
         r.trans_tab = dtt + (size_t)s * nb;
-        r.ky2 = tb.ky2;
-        r.k2max = tb.k2max;
+        r.blo = tb.band.lo, r.bhi = tb.band.hi;
         r.prune = (s == 0) ? 2 : 3;
         if (tu) r.wpb = tu->row_wpb, r.plan = tu->row_plan;
         if (s == 0) {
@@ -1028,6 +1037,7 @@ int batch_class(msx_ctx ctx, const msx_job* jobs, std::vector<BatchItem>& g, std
         c.kx2 = tb.kx2;
         c.ky2 = tb.ky2;
         c.k2max = tb.k2max;
+        c.blo = tb.band.lo, c.bhi = tb.band.hi;
         c.tile = tu ? tu->col_tile : 0;
         if (tu) c.plan = tu->col_plan;
         // one propagator for every running wave (frozen-phonon configurations
@@ -1052,8 +1062,7 @@ int batch_class(msx_ctx ctx, const msx_job* jobs, std::vector<BatchItem>& g, std
             RowArgs<C> f = row_args<C>(w + (long long)active[s + 1] * img, nx, done, twy);
             if (tu) f.plan = tu->row_plan;  // the single-job loop's final sweep
             f.scale = inv;
-            f.ky2 = tb.ky2;
-            f.k2max = tb.k2max;
+            f.blo = tb.band.lo, f.bhi = tb.band.hi;
             f.prune = 1;
             LAUNCH_ROW(ny, kRowInv, f);
         }
@@ -1543,7 +1552,9 @@ int partial_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_
     // ky2 >= k2max were not written by the slice loop: neither is touched
     const float k2p = std::min(tb.k2max, std::nextafter(kap_hi, INFINITY));
     // fractions of live columns (for the profiler's byte counts)
-    const double band_slice = ctx->band, band_lens = band_fraction(k2_table(ny, st->by).data(), ny, k2p);
+    const std::vector<float> ky2 = k2_table(ny, st->by);
+    const Band bandp = band_limits(ky2.data(), ny, k2p);
+    const double band_slice = ctx->band, band_lens = band_fraction(ky2.data(), ny, k2p);
     const double scale = 1.0 / ((double)nang * wsum);
     for (int a0 = 0; a0 < nang; a0 += batch) {
         const int nb = std::min(batch, nang - a0);
@@ -1562,6 +1573,7 @@ int partial_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_
             c.kx2 = tb.kx2;
             c.ky2 = tb.ky2;
             c.k2max = k2p;
+            c.blo = bandp.lo, c.bhi = bandp.hi;
             c.ax = st->ax;
             c.by = st->by;
             c.chi1 = M_PI * lam;
@@ -1580,8 +1592,7 @@ int partial_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_
             // intensity summed over the steps per wave
             RowArgs<C> r = row_args<C>(w2, nx, nb, twy);
             r.scale = (Re)1 / ((Re)nx * (Re)nx * (Re)ny);
-            r.ky2 = tb.ky2;
-            r.k2max = k2p;
+            r.blo = bandp.lo, r.bhi = bandp.hi;
             r.prune = 1;
             r.inten = ib;
             r.iacc = d == 0 ? 1 : 2;

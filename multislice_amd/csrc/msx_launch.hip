@@ -129,17 +129,14 @@ hipError_t col_go_tw(const ColArgs<C>& a0, hipStream_t s) {
     // limit (a launch asking for the full 160 KiB is refused)
     constexpr bool DB = MSX_COL_DB && 2 * tile <= 150 * 1024;
     auto k = col_sweep<C, kN, IN, OUT, TW, OPS, DB, PV>;
-    size_t smem = col_list_offset<C, kN, TW, DB>();  // exchange tiles, detector reduction scratch
+    constexpr size_t smem = col_lds_bytes<C, kN, TW, DB>();
+    hipError_t e = set_smem(k, smem);
+    if (e != hipSuccess) return e;
     unsigned grid;
     if (a.wpb <= 0 || (OPS & kColJobs) != 0) {
         // balanced schedule (the built-in one, and the only one of uneven
-        // jobs): -wpb work-groups per resident
-        // slot (0: one), each with its list of (group, live mask) pairs after
-        // the exchange tiles
+        // jobs): -wpb work-groups per resident slot (0: one)
         a.wpb = a.wpb < 0 ? a.wpb : -1;
-        smem += (size_t)groups * sizeof(int2);
-        hipError_t e = set_smem(k, smem);
-        if (e != hipSuccess) return e;
         static std::atomic<long long> cache[kDev];
         long long slots = 0;
         e = resident_groups(k, kTc<PV> * TW, smem, cache, &slots);
@@ -149,8 +146,6 @@ hipError_t col_go_tw(const ColArgs<C>& a0, hipStream_t s) {
     } else {
         const long long nchunk = (a.nb + a.wpb - 1) / a.wpb;
         grid = (unsigned)(groups * nchunk);
-        hipError_t e = set_smem(k, smem);
-        if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(k, dim3(grid), dim3(kTc<PV> * TW), smem, s, a);
     return hipGetLastError();

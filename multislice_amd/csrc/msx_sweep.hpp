@@ -101,11 +101,12 @@ template <typename C> struct RowArgs {
     Re* inten;              // optional |psi|^2 output [nb][nx][N] (after the pointwise stage)
     int nx, nb;
     int wpb;                // waves handled by one work-group (loop with prefetch)
-    // band pruning along y: element iy is "out of band" when ky2[iy] >= k2max.
+    // band pruning along y: element iy is in band when iy < blo or iy >= N - bhi
+    // (the host's test of freqn's ky2 table, which rises with |ky|; bounds in the
+    // arguments cost no loads before the row's own).
     // prune & 1: out-of-band inputs are known to be exactly zero (not loaded);
     // prune & 2: out-of-band outputs are never read (not stored).
-    const float* ky2;
-    float k2max;
+    int blo, bhi;
     int prune;
     // with inten set: iacc 0 writes |psi|^2, 1 writes iw*|psi|^2, 2 adds
     // iw*|psi|^2 to what inten holds (weighted sums over several launches)
@@ -160,7 +161,7 @@ __global__ __launch_bounds__((RowPlanSel<N, PV>::type::T * LPW)) void row_sweep(
     if (p.prune) {
         inb = 0u;
 #pragma unroll
-        for (int e = 0; e < E; ++e) inb |= (p.ky2[t + e * T] < p.k2max ? 1u : 0u) << e;
+        for (int e = 0; e < E; ++e) inb |= (t + e * T < p.blo || t + e * T >= N - p.bhi ? 1u : 0u) << e;
     }
     const unsigned ld_mask = (p.prune & 1) ? inb : ~0u;
     const unsigned st_mask = (p.prune & 2) ? inb : ~0u;
@@ -349,9 +350,10 @@ template <typename C> struct ColArgs {
     int ny, nb, ops;
     int wpb;               // > 0: waves per work-group (chunked); < 0: balanced schedule (below)
     int tile;              // columns per work-group (0: the built-in width for this length)
-    // prune != 0: columns with ky2[iy] >= k2max are skipped entirely (their
-    // k-space values are all masked to zero, so nothing downstream reads them)
-    int prune;
+    // prune != 0: columns out of band (ky2[iy] >= k2max) are skipped entirely
+    // (their k-space values are all masked to zero, so nothing downstream reads
+    // them); the columns in band are iy < blo and iy >= ny - bhi
+    int prune, blo, bhi;
     // oblique cell (kColObl): x = fx / obl_asg, y = fy / obl_bsg (a sin gam,
     // b sin gam), s = x (x - obl_2c y) + y^2 (obl_2c = 2 cos gam), kept where
     // s < obl_smax with the factor exp(-i (obl_pl s - obl_tx x - obl_ty y))
@@ -410,10 +412,9 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblk) {
     const int xcd = bid % kXcd, idx = bid / kXcd;
     return xcd * per + min(xcd, rem) + idx;
 }
-// Byte offset of the balanced schedule's group list in the column sweep's
-// dynamic LDS: after the exchange buffers (which also hold the detector
-// reduction scratch, at least 2 KiB).
-template <typename C, int N, int TW, bool DB> constexpr size_t col_list_offset() {
+// Bytes of the column sweep's dynamic LDS: the exchange buffers, which also
+// hold the detector reduction scratch (at least 2 KiB).
+template <typename C, int N, int TW, bool DB> constexpr size_t col_lds_bytes() {
     constexpr size_t tile = (size_t)N * (TW + 1) * sizeof(C);
     constexpr size_t x = DB ? 2 * tile : tile;
     return x < 2048 ? 2048 : x;
@@ -436,7 +437,6 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
     using PL = typename ColPlanSel<N, PV>::type;
     constexpr int T = PL::T, E = N / T;
     constexpr bool WAVE = false;  // a column is spread over several wavefronts
-    static_assert(TW <= 32, "live-column masks are 32 bits");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     C* smem = reinterpret_cast<C*>(smem_raw);
     const int lw = threadIdx.x % TW, t = threadIdx.x / TW;
@@ -447,60 +447,32 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
     // renumber them so that consecutive logical groups (neighbouring columns,
     // which share L2 lines when TW*sizeof(C) < 128 B) run on the same XCD.
     const int bid = MSX_XCD_REMAP ? xcd_remap((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
-    // bit c set: column gg*TW + c exists and is in band (or pruning is off).
+    // Columns in band (all without pruning) and the groups that hold one: the
+    // first gl groups and those from gr on, ngl in all.  Computed, not listed:
+    // building a list in LDS from the ky2 table cost two memory round trips and
+    // two barriers before the first load (with the row sweep's own ky2 loads,
+    // 23.0 against 20.7 us per slice of a single 256^2 wave).
     // Dead lanes of a partly live group load from the group's first live
     // column (same cache lines as a live lane); their column is transformed
     // on its own, never stored and left out of the detector sums, so the
     // values need no zeroing.
-    auto live_mask = [&](int gg) -> unsigned {
-        unsigned m = 0;
-        for (int c = 0; c < TW; ++c) {
-            const int y = gg * TW + c;
-            if (y < p.ny && (!p.prune || p.ky2[y] < p.k2max)) m |= 1u << c;
-        }
-        return m;
-    };
+    const int blo = p.prune ? p.blo : p.ny, bhi = p.prune ? p.ny - p.bhi : p.ny;  // live: y < blo or y >= bhi
+    const int gl = min((blo + TW - 1) / TW, groups), gr = max(bhi / TW, gl);
+    const int ngl = gl + max(groups - gr, 0);
+    auto live_col = [&](int y) { return y < p.ny && (y < blo || y >= bhi); };
+    // the group's first live column (relative)
+    auto first_live = [&](int gg) { return gg < gl ? 0 : max(bhi - gg * TW, 0); };
     constexpr bool jobs = (OPS & kColJobs) != 0;
     const bool bal = jobs || p.wpb < 0;
-    int2* glist = reinterpret_cast<int2*>(smem_raw + col_list_offset<C, N, TW, DB>());
-    int ngl = 0, gfix = 0, b0 = 0, b1 = 0;
-    unsigned mfix = 0;
+    int gfix = 0, b0 = 0, b1 = 0;
     if (bal) {
-        // stable partition of the groups: the live ones (group, mask) in
-        // ascending order at the front, the dead ones after them
-        __shared__ int cnt[2][16];
-        const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nwv = (blockDim.x + 63) >> 6;
-        int nd = 0;
-        for (int base = 0; base < groups; base += blockDim.x) {
-            const int gg = base + threadIdx.x;
-            const unsigned m = gg < groups ? live_mask(gg) : 0u;
-            const bool lv = m != 0, dd = gg < groups && m == 0;
-            const unsigned long long bl = __ballot(lv), bd = __ballot(dd);
-            if (lane == 0) {
-                cnt[0][wv] = __popcll(bl);
-                cnt[1][wv] = __popcll(bd);
-            }
-            __syncthreads();
-            int pl = ngl, pd = nd, tl = ngl, td = nd;
-            for (int w = 0; w < nwv; ++w) {
-                if (w < wv) pl += cnt[0][w], pd += cnt[1][w];
-                tl += cnt[0][w], td += cnt[1][w];
-            }
-            const unsigned long long below = (1ull << lane) - 1ull;
-            if (lv) glist[pl + __popcll(bl & below)] = make_int2(gg, (int)m);
-            if (dd) glist[groups - 1 - (pd + __popcll(bd & below))] = make_int2(gg, 0);
-            __syncthreads();
-            ngl = __builtin_amdgcn_readfirstlane(tl);  // uniform (LDS sums of ballots)
-            nd = __builtin_amdgcn_readfirstlane(td);
-        }
         if constexpr ((OPS & kColDetect) != 0) {
             // the dead groups' detector partials are zero
+            const int nd = groups - ngl;
             const long long V = (long long)nd * p.nb;
             if ((int)threadIdx.x < p.ndet)
-                for (long long v = bid; v < V; v += gridDim.x) {
-                    const int gd = glist[ngl + (int)(v % nd)].x;
-                    p.partial[((long long)threadIdx.x * p.nb + v / nd) * groups + gd] = 0.0;
-                }
+                for (long long v = bid; v < V; v += gridDim.x)
+                    p.partial[((long long)threadIdx.x * p.nb + v / nd) * groups + gl + (int)(v % nd)] = 0.0;
         }
         if (ngl == 0 || (long long)bid >= (long long)ngl * p.nb) return;
     } else {
@@ -508,8 +480,7 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
         const int chunk = bid / groups;
         b0 = chunk * p.wpb;
         b1 = min(p.nb, b0 + p.wpb);
-        mfix = live_mask(gfix);
-        if (mfix == 0) {
+        if (gfix >= gl && gfix < gr) {
             // whole group outside the band: its detector partials are zero
             if constexpr ((OPS & kColDetect) != 0) {
                 if ((int)threadIdx.x < p.ndet)
@@ -518,8 +489,9 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
             return;
         }
     }
-    // unit i of this work-group: (group, live mask, wave); false past the end
-    const long long units = (long long)ngl * p.nb;
+    // unit i of this work-group: (group, wave); false past the end.  At most
+    // ny * nb of them, below 2^31 for any batch that fits the device memory.
+    const unsigned units = (unsigned)ngl * (unsigned)p.nb;
     // device-side work queue (kColJobs), one counter per XCD: the units of
     // the balanced schedule's later rounds that fall to an XCD's work-groups
     // (consecutive column groups, whose shared cache lines then meet in that
@@ -547,21 +519,19 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
     auto claim_unit = [&](unsigned k) -> unsigned {
         return (1u + k / (unsigned)q_w) * gridDim.x + (unsigned)q_base + k % (unsigned)q_w;
     };
-    auto unit = [&](int i, int& g, unsigned& m, int& b) -> bool {
+    auto unit = [&](int i, int& g, int& b) -> bool {
         if (bal) {
-            long long u = bid + (long long)i * gridDim.x;
+            unsigned u = (unsigned)bid + (unsigned)i * gridDim.x;
             if constexpr (jobs) {
-                if (i > 0) u = (long long)__builtin_amdgcn_readfirstlane(qslot[i & 1]);
+                if (i > 0) u = __builtin_amdgcn_readfirstlane(qslot[i & 1]);
             }
             if (u >= units) return false;
-            const int2 e = glist[(int)(u % ngl)];
-            g = __builtin_amdgcn_readfirstlane(e.x);
-            m = (unsigned)__builtin_amdgcn_readfirstlane(e.y);
-            b = (int)(u / ngl);
+            const int k = (int)(u % (unsigned)ngl);
+            g = k < gl ? k : k - gl + gr;
+            b = (int)(u / (unsigned)ngl);
             return true;
         }
         g = gfix;
-        m = mfix;
         b = b0 + i;
         return b < b1;
     };
@@ -609,8 +579,8 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
     // (the prefetch past a work-group's last unit, issued without a branch).
     const unsigned ostep = (unsigned)T * (unsigned)p.ny;
     const int img_bytes = N * p.ny * (int)sizeof(C);
-    auto load = [&](int g, unsigned m, int b, bool valid, C (&v)[E]) {
-        const int ld_col = ((m >> lw) & 1u) ? lw : __ffs(m) - 1;
+    auto load = [&](int g, int b, bool valid, C (&v)[E]) {
+        const int ld_col = live_col(g * TW + lw) ? lw : first_live(g);
         const C* img = p.psi + (long long)__builtin_amdgcn_readfirstlane(b) * N * p.ny;
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<C*>(img), 0,
                                                                              valid ? img_bytes : 0, kBufWord3);
@@ -620,8 +590,7 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
     };
 
     int g, b;
-    unsigned m;
-    unit(0, g, m, b);  // every work-group that gets here has a unit
+    unit(0, g, b);  // every work-group that gets here has a unit
     if constexpr (jobs) {
         if (threadIdx.x == 0) qslot[1] = claim_unit(atomicAdd(q_ctr, 1u));
         lds_barrier();
@@ -632,7 +601,7 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
     // the next unit never waits for them)
     const C* pnext = nullptr;
     if constexpr (jobs) pnext = p.prop_tab[b];
-    if (MSX_COL_PREFETCH && !gen) load(g, m, b, true, a);
+    if (MSX_COL_PREFETCH && !gen) load(g, b, true, a);
     // Drain the constant loads (and the first tile) once: the wait counters
     // count in issue order, and a load still pending at the loop entry makes
     // the compiler wait for everything issued after it (the prefetch) in
@@ -640,9 +609,7 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
     __builtin_amdgcn_s_waitcnt(0);
     for (int i = 0;; ++i) {
         int g2 = g, b2 = b;
-        unsigned m2 = m;
-        const bool more = unit(i + 1, g2, m2, b2);
-        if (!more) g2 = g, m2 = m, b2 = b;
+        const bool more = unit(i + 1, g2, b2);
         // the claim of unit i+2, issued before the prefetch so that reading
         // its result at the end of this unit never waits for the prefetch
         unsigned claim = 0;
@@ -669,12 +636,12 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
             // unconditional (past the last unit an empty descriptor reads
             // nothing): a branch around the loads would make the compiler
             // wait for them at the join
-            if (!gen) load(g2, m2, b2, more, nxt);
+            if (!gen) load(g2, b2, more, nxt);
         } else {
-            if (!gen) load(g, m, b, true, a);
+            if (!gen) load(g, b, true, a);
         }
         const int iy = col_y(g);
-        const bool live = (m >> lw) & 1u;
+        const bool live = live_col(g * TW + lw);
         const double ky = (gen || (OPS & kColCtf)) ? (double)freq_index(iy, p.ny) / p.by : 0.0;
         const double oy = (OPS & kColObl) ? (double)freq_index(iy, p.ny) / p.obl_bsg : 0.0;
         if constexpr (gen) {
@@ -798,7 +765,6 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
             for (int e = 0; e < E; ++e) a[e] = nxt[e];
         }
         g = g2;
-        m = m2;
         b = b2;
     }
 }
