@@ -17,6 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libmsx.so")
 SIZES = [16, 32, 64, 128, 256, 384, 512, 768, 1024, 2048]
+LOOP_SIZES = [128, 256, 384, 512]  # rows of the persistent slice loop
 ARCH = os.environ.get("MSX_OFFLOAD_ARCH", "gfx950")
 
 
@@ -54,6 +55,8 @@ def build(jobs=None, verbose=True, defines=(), out=None, bdir=None):
     for n in SIZES:
         units.append((os.path.join(CSRC, "msx_launch.hip"), os.path.join(bdir, f"launch_{n}.o"),
                       [f"-DMSX_N={n}"]))
+    for n in LOOP_SIZES:
+        units.append((os.path.join(CSRC, "msx_loop.hip"), os.path.join(bdir, f"loop_{n}.o"), [f"-DMSX_N={n}"]))
     for name in ("msx_potential", "msx_api", "msx_unet", "msx_unet_kernels", "msx_specimen", "msx_formats",
                  "msx_binning", "msx_lms", "msx_series"):
         units.append((os.path.join(CSRC, name + ".hip"), os.path.join(bdir, name + ".o"), []))

@@ -86,6 +86,37 @@ template <typename C> void col_tiles(int nx, int* def, int* alt) {
 #undef MSX_CASE
 }
 
+// persistent slice loop (msx_loop.hip), lengths 128 to 512 on both axes
+#define MSX_FOR_EACH_LOOP(X) X(128) X(256) X(384) X(512)
+template <typename C> struct LoopArgs;
+#define MSX_DECL_LOOP(NN)                                                                     \
+    template <typename C> hipError_t loop_prepare_##NN(int nx, int* units, int* resident);    \
+    template <typename C> hipError_t launch_loop_##NN(int nx, const LoopArgs<C>& a, int teams, hipStream_t s);
+MSX_FOR_EACH_LOOP(MSX_DECL_LOOP)
+#undef MSX_DECL_LOOP
+inline bool loop_built(int nx, int ny) {
+    bool x = false, y = false;
+#define MSX_CASE(NN) x |= nx == NN, y |= ny == NN;
+    MSX_FOR_EACH_LOOP(MSX_CASE)
+#undef MSX_CASE
+    return x && y;
+}
+// work-groups that a wave's row phase can use, and that are resident at once
+template <typename C> hipError_t loop_prepare(int nx, int ny, int* units, int* resident) {
+#define MSX_CASE(NN) \
+    if (ny == NN) return loop_prepare_##NN<C>(nx, units, resident);
+    MSX_FOR_EACH_LOOP(MSX_CASE)
+#undef MSX_CASE
+    return hipErrorInvalidValue;
+}
+template <typename C> hipError_t launch_loop(int nx, int ny, const LoopArgs<C>& a, int teams, hipStream_t s) {
+#define MSX_CASE(NN) \
+    if (ny == NN) return launch_loop_##NN<C>(nx, a, teams, s);
+    MSX_FOR_EACH_LOOP(MSX_CASE)
+#undef MSX_CASE
+    return hipErrorInvalidValue;
+}
+
 // potential splat (msx_potential.hip)
 struct AtomRec {
     double x, y;   // Angstrom, wrapped into [0,a) x [0,b)

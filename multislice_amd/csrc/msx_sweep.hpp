@@ -52,13 +52,17 @@ constexpr int kMaxDet = 8;
 // 4 GiB.
 constexpr int kBufWord3 = 0x00020000;
 constexpr unsigned kBufDrop = 0x80000000u;
-__device__ __forceinline__ void buf_store(float2 v, __amdgpu_buffer_rsrc_t r, unsigned off) {
+// AUX: cache policy bits; kScopeDev (sc1) makes a load or store coherent over
+// the whole device (past the XCD's own caches) for data that work-groups of
+// one kernel exchange.
+constexpr int kScopeDev = 16;
+template <int AUX = 0> __device__ __forceinline__ void buf_store(float2 v, __amdgpu_buffer_rsrc_t r, unsigned off) {
     using u2 = __attribute__((ext_vector_type(2))) unsigned;
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, (int)off, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, (int)off, 0, AUX);
 }
-__device__ __forceinline__ void buf_store(double2 v, __amdgpu_buffer_rsrc_t r, unsigned off) {
+template <int AUX = 0> __device__ __forceinline__ void buf_store(double2 v, __amdgpu_buffer_rsrc_t r, unsigned off) {
     using u4 = __attribute__((ext_vector_type(4))) unsigned;
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, (int)off, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), r, (int)off, 0, AUX);
 }
 __device__ __forceinline__ void buf_store(float v, __amdgpu_buffer_rsrc_t r, unsigned off) {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)off, 0, 0);
@@ -69,18 +73,11 @@ __device__ __forceinline__ void buf_store(double v, __amdgpu_buffer_rsrc_t r, un
 }
 // Raw buffer loads: an offset at or beyond the descriptor's size reads zero
 // without touching memory.
-template <typename C> __device__ __forceinline__ C buf_load(__amdgpu_buffer_rsrc_t r, unsigned off);
-template <> __device__ __forceinline__ float buf_load<float>(__amdgpu_buffer_rsrc_t r, unsigned off) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
-}
-template <> __device__ __forceinline__ double buf_load<double>(__amdgpu_buffer_rsrc_t r, unsigned off) {
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
-}
-template <> __device__ __forceinline__ float2 buf_load<float2>(__amdgpu_buffer_rsrc_t r, unsigned off) {
-    return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
-}
-template <> __device__ __forceinline__ double2 buf_load<double2>(__amdgpu_buffer_rsrc_t r, unsigned off) {
-    return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
+template <typename C, int AUX = 0> __device__ __forceinline__ C buf_load(__amdgpu_buffer_rsrc_t r, unsigned off) {
+    if constexpr (sizeof(C) == 4) return __builtin_bit_cast(C, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, AUX));
+    else if constexpr (sizeof(C) == 8)
+        return __builtin_bit_cast(C, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, AUX));
+    else return __builtin_bit_cast(C, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, AUX));
 }
 
 // sin and cos in FP32 for |x| <= kSincosMax: reduction by n pi/2 in three fused
