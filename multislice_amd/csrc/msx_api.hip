@@ -1919,6 +1919,7 @@ int splat_binned(msx_ctx ctx, RadArgs& ra, const BinGeom& g, int nx, int ny, dou
     sa.rtab = nullptr;
     sa.rcoef = nullptr;
     sa.rt_noct = 0;
+    sa.nsp = ra.nsp;
     if (prec == MSX_F32 && ra.nsp > 0) {
         // FP32 output: V_Z(r^2) from radial tables (below FP32 resolution of
         // the exact sum, which the FP64 output keeps); octaves from 2^kRadOmin

@@ -145,10 +145,14 @@ struct SplatArgs {
     int nx, ny, nslices, nbx, nby, table, formula;
     const double* rtab;      // radial tables [nsp][rt_noct * (kRadPts + 3) + 1] (FP32 output), or nullptr: exact
     const double2* rcoef;    // their interval coefficients [nsp][rt_noct * kRadPts][2]
-    int rt_noct;
+    int rt_noct, nsp;
     // filled by launch_splat: pixel and bin widths (a / nx, b / ny, a / nbx,
-    // b / nby; IEEE division on the host gives the kernel's own quotients)
+    // b / nby; IEEE division on the host gives the kernel's own quotients); for
+    // the tile kernel tiles along y and in all, tiles per wavefront, the table
+    // intervals [ilo, ilo + nint) that LDS holds and what turns the top bits of
+    // r^2 into a position among them
     double dx, dy, bwx, bwy;
+    int ty, tiles, each, ilo, nint, ibase;
 };
 struct RadArgs {
     double* tab;    // [nsp][noct * (kRadPts + 3) + 1]

@@ -12,6 +12,9 @@
 //    distances in float), which removes the small-r rounding of K0's log.
 // The per-pixel contribution rule is the reference's: minimum image per axis,
 // r < radius, r clamped >= 1e-10, formula and table selectable.
+#include <algorithm>
+#include <cmath>
+
 #include "msx_internal.h"
 #include "msx_philox.h"
 #include "fparams_tables.inc"
@@ -351,12 +354,271 @@ __global__ __launch_bounds__(256) void splat_kernel(SplatArgs p) {
     }
 }
 
+// The same sum for a large FP32 potential, with the table intervals that nearly
+// all pairs use in LDS.  A pair reads 32 bytes of coefficients at an interval of
+// its own: through the vector cache that is a line per lane, and the kernel
+// above spends most of its time on it (2048^2 x 24 slices, 162240 atoms of three
+// species, radius 3 A: whole call 1236 us).  Pairs are spread evenly over r^2, so the top
+// kSplatInt / nsp intervals below radius^2 hold all but a few percent of them;
+// 16 wavefronts share them, one work-group per CU, and lanes below read memory.
+// A wavefront is a tile of 16 columns by 32 rows by itself, two by two blocks of
+// 8 columns by 16 rows, two pixels per lane and block.  It takes the atoms of
+// the bins in the order of the kernel above, 64 at a time, one per lane; each
+// lane finds which blocks its atom can reach (a conservative bound on the
+// distance from the atom to the block), and the atoms that reach any are read
+// out lane by lane into scalar registers and summed by those blocks: the same
+// pairs in the same order, the same bits.  A wavefront takes the slices of one
+// place after the other: bin bounds and pixel positions are set up once, and
+// the next slice's runs are loaded ahead.  848 us; vector instructions and the
+// LDS pipe (bank conflicts included) are then each busy about two thirds of the
+// time.  With the tables in memory the call took 1200 us; loads a block ahead
+// spilled (1180 us); 12 or 8 wavefronts were slower.
+constexpr int kTileThreads = 1024, kTileX = 16, kTileY = 32;
+// table intervals of all species that LDS holds: (c0, c1) in one array, (c2, c3)
+// in a second one within reach of the LDS instructions' 16-bit offset
+constexpr int kSplatInt = 3840;
+
+__device__ __forceinline__ double readlane_f64(double v, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
+__global__ __launch_bounds__(kTileThreads) void splat_tile_kernel(SplatArgs p) {
+    constexpr int NS = 2, NB = NS * NS;  // blocks per axis, per tile
+    // [nsp][nint] (c0, c1), then the same of (c2, c3)
+    __shared__ double2 ltab[2 * kSplatInt];
+    for (int sp = 0; sp < p.nsp; ++sp) {
+        const double2* q = p.rcoef + 2ll * ((long long)sp * p.rt_noct * kRadPts + p.ilo);
+        for (int i = threadIdx.x; i < 2 * p.nint; i += kTileThreads)
+            ltab[(i & 1) * kSplatInt + sp * p.nint + (i >> 1)] = q[i];
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int wave = blockIdx.x * (kTileThreads / 64) + wv;
+    const double dx = p.dx, dy = p.dy, r2max = p.radius * p.radius;
+    // block half extents and the reach (cutoff plus a margin far above rounding)
+    const double hx = 3.5 * dx, hy = 7.5 * dy, reach2 = (p.radius + 1e-6) * (p.radius + 1e-6);
+    // the image test: no pixel of the tile takes an atom's periodic image on
+    // an axis where the atom's distance to the tile centre plus the tile's
+    // half extent stays below half the period (margin far above rounding)
+    constexpr double tx = 0.5 * (kTileX - 1), ty = 0.5 * (kTileY - 1);
+    const double gx = 0.5 * p.a * (1.0 - 1e-9) - tx * dx, gy = 0.5 * p.b * (1.0 - 1e-9) - ty * dy;
+    const long long cstride = 2ll * p.rt_noct * kRadPts;
+    const long long tstride = (long long)p.rt_noct * (kRadPts + 3) + 1;
+    // the wavefront's tiles: slices of one place after the other
+    int tile = wave * p.each;
+    const int tend = min(tile + p.each, p.tiles);
+    while (tile < tend) {
+        int kz = tile % p.nslices;
+        const int place = tile / p.nslices, kend = min(p.nslices, kz + tend - tile);
+        tile += kend - kz;
+        const int x0 = (place / p.ty) * kTileX, y0 = (place % p.ty) * kTileY;
+        const int iy0 = y0 + (lane & 7), ix0 = x0 + (lane >> 3);
+        double xp[NS], yp[2 * NS];
+#pragma unroll
+        for (int j = 0; j < NS; ++j) xp[j] = (ix0 + 8 * j) * dx;
+#pragma unroll
+        for (int j = 0; j < 2 * NS; ++j) yp[j] = (iy0 + 8 * j) * dy;
+        // bins reached by this tile: floor((t d -/+ radius) / w) for its first and
+        // last pixel t on each axis, one bound per lane (lanes 0-3: x low, x high,
+        // y low, y high)
+        const bool ly = (lane & 2) != 0, lhi = (lane & 1) != 0;
+        const int tl = ly ? y0 + (lhi ? kTileY - 1 : 0) : x0 + (lhi ? kTileX - 1 : 0);
+        const double el = (double)tl * (ly ? dy : dx) + (lhi ? p.radius : -p.radius);
+        const int ql = (int)floor(el / (ly ? p.bwy : p.bwx));
+        int bxa = __builtin_amdgcn_readlane(ql, 0), bxb = __builtin_amdgcn_readlane(ql, 1);
+        int bya = __builtin_amdgcn_readlane(ql, 2), byb = __builtin_amdgcn_readlane(ql, 3);
+        if (bxb - bxa + 1 >= p.nbx) { bxa = 0; bxb = p.nbx - 1; }
+        if (byb - bya + 1 >= p.nby) { bya = 0; byb = p.nby - 1; }
+        // the first bin column and row wrapped into the cell (lanes 0 and 1)
+        const int vl = (lane & 1) ? bya : bxa, ml = (lane & 1) ? p.nby : p.nbx;
+        int wl = vl % ml;
+        if (wl < 0) wl += ml;
+        const int bxw_a = __builtin_amdgcn_readlane(wl, 0), byw_a = __builtin_amdgcn_readlane(wl, 1);
+        // bin rows of the two runs of every column: bya up to the wrap, then
+        // from row 0
+        const int len1 = min(byb - bya + 1, p.nby - byw_a), len2 = byb - bya + 1 - len1;
+        const int nrows = (lane & 1) ? len2 : len1, row0 = (lane & 1) ? 0 : byw_a;
+        // run j of a group of kSplatCols columns (column g0 + j / 2, part j % 2) in
+        // lane j: its first atom and the one past its last
+        auto load_runs = [&](int z, int g0) -> int2 {
+            if (lane >= 2 * min(kSplatCols, bxb - g0 + 1) || nrows <= 0) return make_int2(0, 0);
+            int bxw = bxw_a + (g0 - bxa) + (lane >> 1);  // < 2 nbx: the range spans at most nbx columns
+            if (bxw >= p.nbx) bxw -= p.nbx;
+            const int cell = (z * p.nbx + bxw) * p.nby + row0;
+            return make_int2(p.cell_start[cell], p.cell_start[cell + nrows]);
+        };
+        const double bcx = x0 * dx + hx, bcy = y0 * dy + hy;
+        const double cx = x0 * dx + tx * dx, cy = y0 * dy + ty * dy;
+        int2 run = load_runs(kz, bxa);
+        for (; kz < kend; ++kz) {
+            double v[2 * NB];
+#pragma unroll
+            for (int j = 0; j < 2 * NB; ++j) v[j] = 0.0;
+            for (int g0 = bxa; g0 <= bxb; g0 += kSplatCols) {
+                const int nrun = 2 * min(kSplatCols, bxb - g0 + 1);
+                const int rst = run.x, rcnt = run.y - run.x;
+                // the next group's runs, or the next slice's, before they are needed
+                if (g0 + kSplatCols <= bxb) run = load_runs(kz, g0 + kSplatCols);
+                else if (kz + 1 < kend) run = load_runs(kz + 1, bxa);
+                int incl = rcnt;
+                for (int o = 1; o < nrun; o <<= 1) {
+                    const int t = __shfl_up(incl, o, 64);
+                    if (lane >= o) incl += t;
+                }
+                const int total = __builtin_amdgcn_readlane(incl, nrun - 1);
+                const int rpos = incl - rcnt, rdel = rst - rpos;  // first position in the list, atom index - position
+                const unsigned long long filled = __ballot(rcnt > 0);
+                for (int base = 0; base < total; base += 64) {
+                    const int g = base + lane;
+                    // the run holding position g: the last filled one starting at or
+                    // before g
+                    int delta = 0;
+                    for (unsigned long long w = filled; w; w &= w - 1) {
+                        const int j = __builtin_ctzll(w);
+                        const int pos = __builtin_amdgcn_readlane(rpos, j), del = __builtin_amdgcn_readlane(rdel, j);
+                        if (g >= pos) delta = del;
+                    }
+                    AtomRec at{};
+                    int tag = 0;  // blocks reached | periodic image possible << 8 | slot << 16
+                    if (g < total) {
+                        at = p.atoms[g + delta];
+                        double qx[NS], qy[NS];
+#pragma unroll
+                        for (int j = 0; j < NS; ++j) {
+                            const double rx = fabs(at.x - (bcx + 8 * j * dx)), ry = fabs(at.y - (bcy + 16 * j * dy));
+                            const double ex = fmax((rx > 0.5 * p.a ? p.a - rx : rx) - hx, 0.0);
+                            const double ey = fmax((ry > 0.5 * p.b ? p.b - ry : ry) - hy, 0.0);
+                            qx[j] = ex * ex;
+                            qy[j] = ey * ey;
+                        }
+#pragma unroll
+                        for (int j = 0; j < NB; ++j)
+                            if (qx[j % NS] + qy[j / NS] <= reach2) tag |= 1 << j;
+                        if (!(fabs(at.x - cx) < gx) || !(fabs(at.y - cy) < gy)) tag |= 1 << 8;
+                    }
+                    unsigned long long todo = __ballot((tag & 255) != 0);
+                    tag |= (int)at.slot << 16;
+                    while (todo) {
+                        const int l = __builtin_ctzll(todo);
+                        todo &= todo - 1;
+                        const double ax = readlane_f64(at.x, l), ay = readlane_f64(at.y, l);
+                        const double occ =
+                            (double)__int_as_float(__builtin_amdgcn_readlane(__float_as_int(at.occ), l));
+                        const int tg = __builtin_amdgcn_readlane(tag, l);
+                        const int slot = tg >> 16, lrow = slot * p.nint;
+#pragma unroll
+                        for (int j = 0; j < NB; ++j) {
+                            if (!(tg & (1 << j))) continue;
+                            double dX = ax - xp[j % NS], dY[2];
+#pragma unroll
+                            for (int m = 0; m < 2; ++m) dY[m] = ay - yp[2 * (j / NS) + m];
+                            if (tg & (1 << 8)) {
+                                dX = fabs(dX);
+                                if (dX >= p.a / 2.0) dX -= p.a;
+#pragma unroll
+                                for (int m = 0; m < 2; ++m) {
+                                    dY[m] = fabs(dY[m]);
+                                    if (dY[m] >= p.b / 2.0) dY[m] -= p.b;
+                                }
+                            }
+                            // V_Z(r2) from the species' table: interval and
+                            // position from the bits of r2.  Every lane reads LDS
+                            // (clamped to the last interval); lanes below its
+                            // intervals then read the table in memory.
+                            double2 c01[2], c23[2];
+                            double r2[2];
+                            int i[2];
+                            bool in[2];
+                            unsigned long long low = 0;
+#pragma unroll
+                            for (int m = 0; m < 2; ++m) {
+                                r2[m] = fma(dX, dX, dY[m] * dY[m]);
+                                in[m] = r2[m] < r2max;
+                                i[m] = (int)((unsigned)__double2hiint(r2[m]) >> 12) - p.ibase;
+                                low |= __ballot(in[m] && i[m] < 0);
+                                const unsigned u = lrow + min((unsigned)i[m], (unsigned)p.nint - 1u);
+                                c01[m] = ltab[u];
+                                c23[m] = ltab[kSplatInt + u];
+                            }
+                            if (low) {
+#pragma unroll
+                                for (int m = 0; m < 2; ++m) {
+                                    if (in[m] && i[m] < 0) {
+                                        const bool cl = r2[m] < 1.0e-20;
+                                        const double2* q = p.rcoef + slot * cstride + 2 * (cl ? 0 : i[m] + p.ilo);
+                                        c01[m] = q[0];
+                                        c23[m] = q[1];
+                                        if (cl) {
+                                            c01[m] = make_double2(p.rtab[slot * tstride + tstride - 1], 0.0);
+                                            c23[m] = make_double2(0.0, 0.0);
+                                        }
+                                    }
+                                }
+                            }
+#pragma unroll
+                            for (int m = 0; m < 2; ++m)
+                                if (in[m]) v[2 * j + m] += occ * rad_cubic(c01[m], c23[m], rad_position((unsigned long long)__double_as_longlong(r2[m])));
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    const int ix = ix0 + 8 * (j % NS), iy = iy0 + 16 * (j / NS) + 8 * m;
+                    if (ix < p.nx && iy < p.ny) {
+                        const long long o = ((long long)kz * p.nx + ix) * p.ny + iy;
+                        p.v32[o] = (float)v[2 * j + m];
+                    }
+                }
+        }
+    }
+}
+
+// From this many pixels the tile kernel is taken, and with at least this many
+// intervals of a species in LDS.  Whole calls, us, per-pixel / tile kernel (0.1 A
+// per pixel, device atoms, radius 3 A and three species but where given): 512^2
+// x 4 125 / 135, x 12 157 / 153, x 16 171 / 160; 1024^2 x 8 222 / 191, of radius
+// 10 A 877 / 555, of 1 A 166 / 146, of one species 218 / 185, of 20 (192
+// intervals) 244 / 230, of 30 (128) 251 / 251 and of 60 (64) 277 / 298; 2048^2 x
+// 8 519 / 387.  Filling LDS and 4096 wavefronts' worth of larger tiles is what
+// the smaller calls do not make up for.
+constexpr long long kTilePixels = 3LL << 20;
+constexpr int kTileIntervals = 192;
+
 hipError_t launch_splat(const SplatArgs& args, hipStream_t s) {
     SplatArgs a = args;
     a.dx = a.a / a.nx;
     a.dy = a.b / a.ny;
     a.bwx = a.a / a.nbx;
     a.bwy = a.b / a.nby;
+    if (a.rtab && (long long)a.nx * a.ny * a.nslices >= kTilePixels && a.nsp <= kSplatInt / kTileIntervals) {
+        const double r2max = a.radius * a.radius;
+        int e;
+        const double f = std::frexp(r2max, &e);  // r2max = 2 f 2^(e - 1), 2 f in [1, 2)
+        // one past the interval of radius^2, the top of those the pairs use
+        const long long top = std::min<long long>((long long)a.rt_noct * kRadPts,
+                                                  (long long)(e - 1 - kRadOmin) * kRadPts +
+                                                      (int)((2.0 * f - 1.0) * kRadPts) + 1);
+        if (top >= kTileIntervals) {
+            a.nint = (int)std::min<long long>(top, kSplatInt / a.nsp);
+            a.ilo = (int)top - a.nint;
+            a.ibase = a.ilo + (1023 + kRadOmin) * kRadPts;
+            a.ty = (a.ny + kTileY - 1) / kTileY;
+            a.tiles = a.ty * ((a.nx + kTileX - 1) / kTileX) * a.nslices;
+            int dev = 0, cus = 0;
+            hipError_t er = hipGetDevice(&dev);
+            if (er == hipSuccess) er = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+            if (er != hipSuccess) return er;
+            const int nwv = kTileThreads / 64;
+            a.each = (a.tiles + cus * nwv - 1) / (cus * nwv);
+            const int wgs = (a.tiles + a.each * nwv - 1) / (a.each * nwv);
+            hipLaunchKernelGGL(splat_tile_kernel, dim3((unsigned)wgs), dim3(kTileThreads), 0, s, a);
+            return hipGetLastError();
+        }
+    }
     dim3 grid((a.ny + kSplatRows - 1) / kSplatRows, (a.nx + 15) / 16, a.nslices);
     if (a.rtab) hipLaunchKernelGGL(splat_kernel<true>, grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL(splat_kernel<false>, grid, dim3(256), 0, s, a);
