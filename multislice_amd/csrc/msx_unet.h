@@ -60,9 +60,19 @@ size_t conv3_pack_size(int M, int C);  // elements of one layer's packed weights
 bool conv3_fits(const ConvArgs& a);    // image small enough for the packed kernel
 hipError_t launch_pack_conv3(const PackArgs& a, int layers, hipStream_t s);
 
-hipError_t launch_conv(int mode, int ks, const ConvArgs& a, hipStream_t s);
-// floats of ConvArgs::partial that launch_conv(kBwdWeight, ks, a) needs (0: none)
+hipError_t launch_conv(int mode, int ks, const ConvArgs& a, hipStream_t s);  // kFwd, kBwdData
+
+// kBwdWeight of several layers at once: the products, one launch for all 3x3
+// layers that wgrad3 takes and one for each other, then one launch that adds
+// their slices and forms the bias gradients.
+constexpr int kMaxWgrad = 24;
+struct WgradLayer {
+    ConvArgs a;
+    int ks;
+};
+// floats of ConvArgs::partial that a layer needs (0: none)
 size_t conv_wgrad_scratch(int ks, const ConvArgs& a);
+hipError_t launch_wgrad(const WgradLayer* layers, int n, hipStream_t s);  // n <= kMaxWgrad
 hipError_t launch_avgpool_fwd(const float* x, float* y, long long nc, int H, int W, hipStream_t s);
 hipError_t launch_avgpool_bwd(const float* gy, float* gx, long long nc, int H, int W, hipStream_t s);
 hipError_t launch_upsample_fwd(const float* x, float* y, int N, int C, int H, int W, int Ct, int c0, hipStream_t s);

@@ -12,6 +12,8 @@
 // where G = dY masked by the ReLU of the layer's output.  Tensors are NCHW FP32.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "msx_fft.hpp"  // lds_barrier
 #include "msx_unet.h"
 
@@ -184,7 +186,7 @@ __global__ __launch_bounds__(256) void conv_gemm(ConvArgs p) {
             }
             if (p.accumulate) *dst += c; else *dst = c;
         } else if (gridDim.z > 1) {
-            // this reduction slice's share of dW[co][ci][tap]; wgrad_reduce
+            // this reduction slice's share of dW[co][ci][tap]; grad_finish
             // adds the slices in order (no atomics: the same sums every run)
             p.partial[(long long)blockIdx.z * M * N + m * N + n] = c;
         } else {
@@ -193,17 +195,40 @@ __global__ __launch_bounds__(256) void conv_gemm(ConvArgs p) {
     }
 }
 
-// The second half of a layer's parameter gradients in one launch.  Work-groups
-// 0 .. nbias - 1: the bias gradient of channel blockIdx.x, per-thread sums over
-// the pixels t, t + 256, .. and a tree.  The others: 256 weights each, adding
-// the reduction slices in order.  Fixed orders: the same sums every run.  Both
-// are chains of additions fed by loads, so the loads run 16 and 32 ahead (one
-// at a time: 13.5 and 14.6 us per layer; 8.9 together now).
-__global__ __launch_bounds__(256) void grad_finish(const float* g, const float* y, int relu, int N, int C, int HW,
-                                                   float* db, int nbias, const float* __restrict__ part, float* dw,
-                                                   long long mn, int splits) {
-    if ((int)blockIdx.x >= nbias) {
-        const long long i = (long long)((int)blockIdx.x - nbias) * 256 + threadIdx.x;
+// What the weight gradient of one layer needs, in a table passed by value: the
+// product kernel's and grad_finish's first work-group of the layer.
+struct WgradItem {
+    const float *x, *g, *y;
+    float *out, *partial, *db;
+    long long mn;  // weights that have slices to add (0: one slice, added by the product)
+    int N, Cin, Cout, H, W, relu, splits, first, finish;
+};
+struct WgradTable {
+    WgradItem item[kMaxWgrad];
+    int n;
+};
+
+// The second half of the layers' parameter gradients in one launch.  Of a
+// layer's work-groups the first Cout: the bias gradient of a channel, per-thread
+// sums over the pixels t, t + 256, .. and a tree.  The others: 256 weights each,
+// adding the reduction slices in order.  Fixed orders: the same sums every run.
+// Both are chains of additions fed by loads, so the loads run 16 and 32 ahead
+// (one at a time: 13.5 and 14.6 us per layer; 8.9 together; the 15 layers of a
+// training step in one launch 36 instead of 132).
+__global__ __launch_bounds__(256) void grad_finish(WgradTable t) {
+    int l = 0;
+    while (l + 1 < t.n && (int)blockIdx.x >= t.item[l + 1].finish) ++l;
+    const WgradItem& q0 = t.item[l];
+    const float* const g = q0.g;
+    const float* const y = q0.y;
+    const float* __restrict__ part = q0.partial;
+    float* const db = q0.db;
+    float* const dw = q0.out;
+    const int N = q0.N, C = q0.Cout, HW = q0.H * q0.W, relu = q0.relu, splits = q0.splits;
+    const int nbias = db ? C : 0, block = (int)blockIdx.x - q0.finish;
+    const long long mn = q0.mn;
+    if (block >= nbias) {
+        const long long i = (long long)(block - nbias) * 256 + threadIdx.x;
         if (i >= mn) return;
         const float* q = part + i;
         float s = 0.f;
@@ -221,7 +246,7 @@ __global__ __launch_bounds__(256) void grad_finish(const float* g, const float* 
         return;
     }
     __shared__ float red[256];
-    const int c = blockIdx.x;
+    const int c = block;
     const long long n = (long long)N * HW;
     float s = 0.f;
     for (long long i0 = threadIdx.x; i0 < n; i0 += 256 * 16) {
@@ -251,6 +276,164 @@ __global__ __launch_bounds__(256) void grad_finish(const float* g, const float* 
         __syncthreads();
     }
     if (threadIdx.x == 0) db[c] = red[0];
+}
+
+// ------------------------------------------------------- 3x3 weight gradient
+// wgrad3: conv_gemm's weight gradient for 3x3 layers whose rows are whole runs
+// of 4 pixels.  conv_gemm gathers every (channel, tap) of a pixel as a scalar
+// with its index arithmetic, about 400 instructions per thread and 32 pixels,
+// and bounds on it (24 us per layer of a 32^2 training step whatever its size).
+// Here a work-group owns 32 output channels x 32 input channels and all 9 taps,
+// one wavefront per row of taps.  Per block of 64 pixels a thread loads 8
+// pixels of a channel and their neighbours left and right as vectors, the next
+// block's while this one is computed, and writes them to LDS as three bf16
+// operands, one per column of taps, so that the matrix cores read whole aligned
+// runs.  Slices of the reduction, the order of pixels and their places in each
+// MFMA are conv_gemm's: every partial sum keeps its bits.  Per layer, us,
+// conv_gemm / wgrad3 (images, input and output channels, size): 16, 96, 32, 32^2
+// 34 / 19; 16, 192, 64, 16^2 44 / 17; 16, 256, 256, 4^2 18 / 13; 16, 64, 64, 64^2
+// 202 / 51; 16, 128, 128, 64^2 715 / 142.  At the small sizes it is bound by
+// latency (load, LDS, 3 dependent MFMAs, store), so layers share a launch: the
+// 14 of a training step of 16 32^2 images 340 us with conv_gemm, 181 one by
+// one, 65 together.
+constexpr int kWB = 64, kWRow = kWB + 8;  // pixels per block; LDS rows of 144 bytes
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(192) void wgrad3(WgradTable t) {
+    int l = 0;
+    while (l + 1 < t.n && (int)blockIdx.x >= t.item[l + 1].first) ++l;
+    const WgradItem p = t.item[l];
+    __shared__ __align__(16) __bf16 tile[10][32][kWRow];
+    __bf16 (*const As)[kWRow] = tile[0];
+    float* const Ds = reinterpret_cast<float*>(&tile[0][0][0]);  // 32 x 288 results at the end, rows of 289
+    static_assert(sizeof(tile) >= 32 * 289 * sizeof(float), "the results reuse the operands' LDS");
+    const int lane = threadIdx.x & 63, ty = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);  // tap row
+    // work-group: input channel tile fastest, then output channel tile, then slice
+    const int ct = (p.Cin + 31) / 32, mt = (p.Cout + 31) / 32, block = (int)blockIdx.x - p.first;
+    const int m0 = block / ct % mt * 32, c0 = block % ct * 32, slice = block / (ct * mt);
+    const int H = p.H, W = p.W, HW = H * W, K = p.N * HW;
+    const int splits = p.splits, chunk = ((K + splits - 1) / splits + BK - 1) / BK * BK;
+    const int k_beg = slice * chunk, k_end = min(k_beg + chunk, K);
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.x), 0, p.Cin * K * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.g), 0, p.Cout * K * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t ry =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.relu ? p.y : p.g), 0, p.Cout * K * 4, 0x00020000);
+    auto load4 = [](__amdgpu_buffer_rsrc_t r, unsigned o) {
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)o, 0, 0));
+    };
+    auto load1 = [](__amdgpu_buffer_rsrc_t r, unsigned o) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)o, 0, 0));
+    };
+    // this lane's 8 pixels of a block: run lane % 8, as two halves of 4 that
+    // each lie in one image row; channels lane / 8 + 8 i
+    const int run = lane & 7, ch = lane >> 3;
+    int k[2], px[2], py[2], pi[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        k[h] = k_beg + 8 * run + 4 * h;
+        pi[h] = k[h] / HW;
+        py[h] = (k[h] - pi[h] * HW) / W;
+        px[h] = k[h] - pi[h] * HW - py[h] * W;
+    }
+    const int qw = kWB / W, rw = kWB - qw * W;
+    f32x4 cx[4][2], ca[2][2], cm[2][2];
+    float cl[4][2], cr[4][2];
+    // loads the block at k[] and steps to the next one
+    auto load = [&] {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const bool in = k[h] < k_end;
+            const int y = py[h] + ty - 1;
+            const bool row = in && (unsigned)y < (unsigned)H;
+            const unsigned bx = (unsigned)((pi[h] * p.Cin + c0 + ch) * HW + y * W + px[h]) * 4u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bool ok = row && c0 + ch + 8 * i < p.Cin;
+                const unsigned o = bx + (unsigned)(8 * i * HW) * 4u;
+                cx[i][h] = load4(rx, ok ? o : 0x80000000u);
+                cl[i][h] = load1(rx, ok && px[h] > 0 ? o - 4u : 0x80000000u);
+                cr[i][h] = load1(rx, ok && px[h] + 4 < W ? o + 16u : 0x80000000u);
+            }
+            const unsigned bg = (unsigned)((pi[h] * p.Cout + m0 + ch) * HW + py[h] * W + px[h]) * 4u;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {  // channel groups ty and ty + 3 (of 4) of the output gradient
+                const int c = ch + 8 * (ty + 3 * i);
+                const bool ok = in && c < 32 && m0 + c < p.Cout;
+                const unsigned o = bg + (unsigned)(8 * (ty + 3 * i) * HW) * 4u;
+                ca[i][h] = load4(rg, ok ? o : 0x80000000u);
+                if (p.relu) cm[i][h] = load4(ry, ok ? o : 0x80000000u);
+            }
+            k[h] += kWB;
+            px[h] += rw;
+            py[h] += qw;
+            if (px[h] >= W) px[h] -= W, ++py[h];
+            while (py[h] >= H) py[h] -= H, ++pi[h];
+        }
+    };
+    f32x16 acc[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[d][v] = 0.f;
+    const int r = lane & 31, kh = (lane >> 5) * 8;
+    load();
+    for (int kb = k_beg; kb < k_end; kb += kWB) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            bf16x8 q[3];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    q[0][4 * h + j] = (__bf16)(j > 0 ? cx[i][h][j > 0 ? j - 1 : 0] : cl[i][h]);
+                    q[1][4 * h + j] = (__bf16)cx[i][h][j];
+                    q[2][4 * h + j] = (__bf16)(j < 3 ? cx[i][h][j < 3 ? j + 1 : 3] : cr[i][h]);
+                }
+#pragma unroll
+            for (int d = 0; d < 3; ++d) *reinterpret_cast<bf16x8*>(&tile[1 + 3 * ty + d][ch + 8 * i][8 * run]) = q[d];
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if (ty + 3 * i > 3) continue;
+            bf16x8 q;
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    q[4 * h + j] = (__bf16)(p.relu && cm[i][h][j] <= 0.f ? 0.f : ca[i][h][j]);
+            *reinterpret_cast<bf16x8*>(&As[ch + 8 * (ty + 3 * i)][8 * run]) = q;
+        }
+        lds_barrier();
+        if (kb + kWB < k_end) load();
+#pragma unroll
+        for (int s = 0; s < kWB; s += 16) {
+            const bf16x8 a = *reinterpret_cast<const bf16x8*>(&As[r][s + kh]);
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const bf16x8 b = *reinterpret_cast<const bf16x8*>(&tile[1 + 3 * ty + d][r][s + kh]);
+                acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[d], 0, 0, 0);
+            }
+        }
+        lds_barrier();
+    }
+    // the 9 taps of 32 input channels are contiguous: through LDS, so that a
+    // wavefront stores whole lines
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            Ds[(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * 289 + 9 * r + 3 * ty + d] = acc[d][v];
+    lds_barrier();
+    const int cols = 9 * min(32, p.Cin - c0);
+    const long long N = 9ll * p.Cin, mn = p.Cout * N;
+    for (int m = ty; m < 32 && m0 + m < p.Cout; m += 3) {
+        const long long o = (m0 + m) * N + 9ll * c0;
+        for (int j = lane; j < cols; j += 64) {
+            const float v = Ds[m * 289 + j];
+            if (splits > 1) p.partial[slice * mn + o + j] = v;
+            else p.out[o + j] += v;
+        }
+    }
 }
 
 // ------------------------------------------------ 3x3 forward and input gradient
@@ -525,6 +708,15 @@ bool conv3_fits(const ConvArgs& a) {
 }
 
 namespace {
+// wgrad3 takes rows of whole, aligned runs of 4 pixels, in tensors that 31-bit
+// byte offsets reach, and at least two blocks of pixels (68 pixels: 13.7 us with
+// conv_gemm, 15.6 with wgrad3; 140: 11 and 9)
+bool wgrad3_fits(const ConvArgs& a) {
+    const long long px = (long long)a.N * a.H * a.W;
+    const uintptr_t at = (uintptr_t)a.x | (uintptr_t)a.g | (a.relu ? (uintptr_t)a.y : 0);
+    return a.W % 4 == 0 && at % 16 == 0 && px >= 2 * kWB && px * std::max(a.Cin, a.Cout) < (1LL << 29);
+}
+
 hipError_t launch_conv3(int mode, const ConvArgs& a, hipStream_t s) {
     const int mt = ((mode == kFwd ? a.Cout : a.Cin) + 31) / 32, pw = mt == 1 ? 4 : (mt <= 3 ? 2 : 1);
     const int tw = pw == 4 ? 16 : 8, th = pw == 1 ? 4 : 8, g = 4 / pw;
@@ -542,13 +734,11 @@ hipError_t launch_conv3(int mode, const ConvArgs& a, hipStream_t s) {
 }
 }  // namespace
 
-hipError_t launch_conv(int mode, int ks, const ConvArgs& a, hipStream_t s) {
+namespace {
+hipError_t launch_conv_gemm(int mode, int ks, const ConvArgs& a, int splits, hipStream_t s) {
     long long M, N, K;
     conv_gemm_shape(mode, ks, a, &M, &N, &K);
     const int bm = conv_bm(M), bn = 4096 / bm;
-    const int splits = mode == kBwdWeight ? wgrad_splits(M, N, K) : 1;
-    if (splits > 1 && !a.partial) return hipErrorInvalidValue;
-    if (a.pack && mode != kBwdWeight) return launch_conv3(mode, a, s);
     dim3 grid((unsigned)((N + bn - 1) / bn), (unsigned)((M + bm - 1) / bm), (unsigned)splits);
 #define MSX_CONV(MODE_, KS_, BM_) hipLaunchKernelGGL((conv_gemm<MODE_, KS_, BM_>), grid, dim3(256), 0, s, a)
 #define MSX_CONV_BM(MODE_, KS_)                    \
@@ -569,12 +759,42 @@ hipError_t launch_conv(int mode, int ks, const ConvArgs& a, hipStream_t s) {
     }
 #undef MSX_CONV_BM
 #undef MSX_CONV
-    if (mode == kBwdWeight && (splits > 1 || a.db)) {
-        const long long mn = splits > 1 ? M * N : 0;
-        const int nbias = a.db ? a.Cout : 0;
-        hipLaunchKernelGGL(grad_finish, dim3((unsigned)(nbias + (mn + 255) / 256)), dim3(256), 0, s, a.g, a.y, a.relu,
-                           a.N, a.Cout, a.H * a.W, a.db, nbias, a.partial, a.out, mn, splits);
+    return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_conv(int mode, int ks, const ConvArgs& a, hipStream_t s) {
+    if (mode == kBwdWeight) return hipErrorInvalidValue;
+    if (a.pack) return launch_conv3(mode, a, s);
+    return launch_conv_gemm(mode, ks, a, 1, s);
+}
+
+hipError_t launch_wgrad(const WgradLayer* layers, int n, hipStream_t s) {
+    if (n < 0 || n > kMaxWgrad) return hipErrorInvalidValue;
+    WgradTable prod{}, fin{};
+    int nprod = 0, nfin = 0;  // work-groups
+    for (int i = 0; i < n; ++i) {
+        const ConvArgs& a = layers[i].a;
+        long long M, N, K;
+        conv_gemm_shape(kBwdWeight, layers[i].ks, a, &M, &N, &K);
+        const int splits = wgrad_splits(M, N, K);
+        if (splits > 1 && !a.partial) return hipErrorInvalidValue;
+        WgradItem q{a.x, a.g, a.y, a.out, a.partial, a.db, splits > 1 ? M * N : 0, a.N, a.Cin, a.Cout, a.H, a.W, a.relu,
+                    splits, nprod, nfin};
+        if (layers[i].ks == 3 && wgrad3_fits(a)) {
+            nprod += ((a.Cout + 31) / 32) * ((a.Cin + 31) / 32) * splits;
+            prod.item[prod.n++] = q;
+        } else {
+            const hipError_t e = launch_conv_gemm(kBwdWeight, layers[i].ks, a, splits, s);
+            if (e != hipSuccess) return e;
+        }
+        if (splits > 1 || a.db) {
+            nfin += (a.db ? a.Cout : 0) + (int)((q.mn + 255) / 256);
+            fin.item[fin.n++] = q;
+        }
     }
+    if (prod.n) hipLaunchKernelGGL(wgrad3, dim3((unsigned)nprod), dim3(192), 0, s, prod);
+    if (fin.n) hipLaunchKernelGGL(grad_finish, dim3((unsigned)nfin), dim3(256), 0, s, fin);
     return hipGetLastError();
 }
 
