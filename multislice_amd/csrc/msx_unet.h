@@ -76,14 +76,16 @@ hipError_t launch_wgrad(const WgradLayer* layers, int n, hipStream_t s);  // n <
 hipError_t launch_avgpool_fwd(const float* x, float* y, long long nc, int H, int W, hipStream_t s);
 hipError_t launch_avgpool_bwd(const float* gy, float* gx, long long nc, int H, int W, hipStream_t s);
 hipError_t launch_upsample_fwd(const float* x, float* y, int N, int C, int H, int W, int Ct, int c0, hipStream_t s);
-hipError_t launch_upsample_bwd(const float* gy, float* gx, int N, int C, int H, int W, int Ct, int c0, hipStream_t s);
+hipError_t launch_cat_bwd(const float* g, float* gup, int C1, float* gskip, int C2, int N, int H, int W,
+                          hipStream_t s);
 hipError_t launch_copy_channels(const float* src, int Cs, int s0, float* dst, int Cd, int d0, int N, int C, int HW,
-                                int accumulate, hipStream_t s);
-hipError_t launch_residual_mse(const float* in, const float* z, const float* t, float* out, float* g, long long n,
-                               float scale, hipStream_t s);
+                                hipStream_t s);
 // y[n][p] = (1/C) sum_c x[n][c][p] (FP32, channels in order)
 hipError_t launch_channel_mean(const float* x, float* y, int N, int C, long long HW, hipStream_t s);
-hipError_t launch_sq_diff(const float* a, const float* b, long long n, double* partial, int nblocks, hipStream_t s);
+hipError_t launch_residual_loss(const float* in, const float* z, const float* t, float* g, long long n, float scale,
+                                double* partial, int nblocks, hipStream_t s);
+// zeros in a and b (b 16-byte aligned, nb a multiple of 4)
+hipError_t launch_clear(float* a, long long na, float* b, long long nb, hipStream_t s);
 hipError_t launch_adam(float* w, const float* gw, float* m, float* v, long long n, float lr, float b1, float b2,
                        float eps, float c1, float c2, hipStream_t s);
 

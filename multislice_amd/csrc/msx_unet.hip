@@ -316,7 +316,7 @@ struct msx_unet_s {
             if (!fused && l < L - 1) {
                 UHIP(launch_avgpool_fwd(eb[l], pl[l], (long long)n * C(l), wh >> l, ww >> l, stream()));
                 UHIP(launch_copy_channels(eb[l], C(l), 0, cat[l], C(l + 1) + C(l), C(l + 1), n, C(l),
-                                          (wh >> l) * (ww >> l), 0, stream()));
+                                          (wh >> l) * (ww >> l), stream()));
             }
         }
         const float* prev = eb[L - 1];
@@ -342,28 +342,26 @@ struct msx_unet_s {
         return MSX_OK;
     }
 
-    // loss = mean (out - t)^2 (out computed here), and every gradient
-    int backward(const float* x, const float* t, double* loss) {
+    // every gradient of mean (out - t)^2, out = the residual + the head's output;
+    // enqueued only, as are the loss's partial sums
+    int backward(const float* x, const float* t) {
         const int L = levels, n = wn;
         const long long cnt = (long long)n * wh * ww;
         UCHK(pack(kBwdData));
         nwg = 0;  // what a failed call may have left
         wg_need = 0;
         // clear the accumulated gradients first: gz is the first tensor of the region
-        UHIP(hipMemsetAsync(grads(), 0, nparam * sizeof(float), stream()));
-        UHIP(hipMemsetAsync(grad_begin, 0, grad_bytes, stream()));
-        UHIP(launch_residual_mse(cin0 > 1 ? xbase : x, z, t, out, gz, cnt, 2.0f / (float)cnt, stream()));
-        UHIP(launch_sq_diff(out, t, cnt, partial, kSqBlocks, stream()));
+        UHIP(launch_clear(grads(), (long long)nparam, grad_begin, (long long)(grad_bytes / sizeof(float)), stream()));
+        UHIP(launch_residual_loss(cin0 > 1 ? xbase : x, z, t, gz, cnt, 2.0f / (float)cnt, partial, kSqBlocks, stream()));
         const float* prev = L > 1 ? db[0] : eb[0];
         float* g_prev = L > 1 ? g_db[0] : g_eb[0];
         UCHK(conv_bwd(head(), 0, prev, z, gz, g_prev));
         for (int l = 0; l <= L - 2; l++) {
-            const int Ct = C(l + 1) + C(l), hl = wh >> l, wl = ww >> l;
+            const int hl = wh >> l, wl = ww >> l;
             UCHK(conv_bwd(dec_b(l), l, da[l], db[l], g_db[l], g_da[l]));
             UCHK(conv_bwd(dec_a(l), l, cat[l], da[l], g_da[l], g_cat[l]));
             float* g_up = (l + 1 <= L - 2) ? g_db[l + 1] : g_eb[L - 1];
-            UHIP(launch_upsample_bwd(g_cat[l], g_up, n, C(l + 1), hl / 2, wl / 2, Ct, 0, stream()));
-            UHIP(launch_copy_channels(g_cat[l], Ct, C(l + 1), g_eb[l], C(l), 0, n, C(l), hl * wl, 1, stream()));
+            UHIP(launch_cat_bwd(g_cat[l], g_up, C(l + 1), g_eb[l], C(l), n, hl / 2, wl / 2, stream()));
         }
         for (int l = L - 1; l >= 0; l--) {
             UCHK(conv_bwd(enc_b(l), l, ea[l], eb[l], g_eb[l], g_ea[l]));
@@ -372,15 +370,19 @@ struct msx_unet_s {
                 UHIP(launch_avgpool_bwd(g_pl[l - 1], g_eb[l - 1], (long long)n * C(l - 1), wh >> (l - 1),
                                         ww >> (l - 1), stream()));
         }
-        UCHK(weight_grads());
+        return weight_grads();
+    }
+
+    // waits for the enqueued work; the loss of the last backward()
+    int finish(double* loss) {
         if (loss) {
-            std::vector<double> h(kSqBlocks);
-            UHIP(hipMemcpyAsync(h.data(), partial, sizeof(double) * kSqBlocks, hipMemcpyDeviceToHost, stream()));
+            double h[kSqBlocks], s = 0.0;
+            UHIP(hipMemcpyAsync(h, partial, sizeof h, hipMemcpyDeviceToHost, stream()));
             UHIP(hipStreamSynchronize(stream()));
-            double s = 0.0;
             for (double v : h) s += v;
-            *loss = s / (double)cnt;
+            *loss = s / (double)((long long)wn * wh * ww);
         }
+        UHIP(hipStreamSynchronize(stream()));
         return MSX_OK;
     }
 };
@@ -602,12 +604,11 @@ MSX_API int msx_unet_gradient(msx_unet net, const float* x, const float* target,
     UCHK(stage_inputs(net, &x, &target, where));
     UCHK(stage_mean(net, x));
     UCHK(net->forward(x));
-    UCHK(net->backward(x, target, loss));
+    UCHK(net->backward(x, target));
     if (grad)
         UHIP(hipMemcpyAsync(grad, net->grads(), net->nparam * sizeof(float),
                             where == MSX_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice, net->stream()));
-    UHIP(hipStreamSynchronize(net->stream()));
-    return MSX_OK;
+    return net->finish(loss);
 }
 
 MSX_API int msx_unet_train_step(msx_unet net, const float* x, const float* target, int n, int h, int w, float lr,
@@ -621,7 +622,7 @@ MSX_API int msx_unet_train_step(msx_unet net, const float* x, const float* targe
     UCHK(stage_inputs(net, &x, &target, where));
     UCHK(stage_mean(net, x));
     UCHK(net->forward(x));
-    UCHK(net->backward(x, target, loss));
+    UCHK(net->backward(x, target));
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     net->step++;
     const float c1 = (float)(1.0 - std::pow((double)b1, (double)net->step));
@@ -629,8 +630,7 @@ MSX_API int msx_unet_train_step(msx_unet net, const float* x, const float* targe
     UHIP(launch_adam(net->params(), net->grads(), net->adam_m(), net->adam_v(), (long long)net->nparam, lr, b1, b2,
                      eps, c1, c2, net->stream()));
     net->weights_changed();
-    UHIP(hipStreamSynchronize(net->stream()));
-    return MSX_OK;
+    return net->finish(loss);  // after the update is enqueued: one wait per step
 }
 
 }  // extern "C"

@@ -826,38 +826,33 @@ __global__ void upsample2_fwd(const float* x, float* y, int N, int C, int H, int
     const int n = (int)(nc / C), c = (int)(nc % C);
     y[(((long long)n * Ct + c0 + c) * Ho + yo) * Wo + xo] = x[((long long)nc * H + yo / 2) * W + xo / 2];
 }
-__global__ void upsample2_bwd(const float* gy, float* gx, int N, int C, int H, int W, int Ct, int c0) {
-    const long long tot = (long long)N * C * H * W;
+// gradient of a concatenation [upsampled (C1) | skip (C2)] of 2H x 2W images:
+// gup[n, c] += the sums over 2x2 of the first C1 channels, gskip += the others
+__global__ void cat_bwd(const float* g, float* gup, int C1, float* gskip, int C2, int N, int H, int W) {
+    const long long t1 = (long long)N * C1 * H * W, t2 = (long long)N * C2 * 4 * H * W;
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= tot) return;
-    const int x = (int)(i % W), y = (int)((i / W) % H);
-    const long long nc = i / ((long long)W * H);
-    const int n = (int)(nc / C), c = (int)(nc % C);
-    const int Wo = 2 * W;
-    const float* s = gy + (((long long)n * Ct + c0 + c) * 2 * H + 2 * y) * Wo + 2 * x;
-    gx[i] += s[0] + s[1] + s[Wo] + s[Wo + 1];
+    const int Wo = 2 * W, Ct = C1 + C2;
+    if (i < t1) {
+        const int x = (int)(i % W), y = (int)((i / W) % H);
+        const long long nc = i / ((long long)W * H);
+        const int n = (int)(nc / C1), c = (int)(nc % C1);
+        const float* s = g + (((long long)n * Ct + c) * 2 * H + 2 * y) * Wo + 2 * x;
+        gup[i] += s[0] + s[1] + s[Wo] + s[Wo + 1];
+    } else if (i < t1 + t2) {
+        const long long j = i - t1, HW = 4LL * H * W, nc = j / HW;
+        const int n = (int)(nc / C2), c = (int)(nc % C2);
+        gskip[j] += g[((long long)n * Ct + C1 + c) * HW + j % HW];
+    }
 }
-// copy channels: dst[n, d0 + c] (+)= src[n, s0 + c], c < C
-__global__ void copy_channels(const float* src, int Cs, int s0, float* dst, int Cd, int d0, int N, int C, int HW,
-                              int accumulate) {
+// copy channels: dst[n, d0 + c] = src[n, s0 + c], c < C
+__global__ void copy_channels(const float* src, int Cs, int s0, float* dst, int Cd, int d0, int N, int C, int HW) {
     const long long tot = (long long)N * C * HW;
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= tot) return;
     const int pix = (int)(i % HW);
     const long long nc = i / HW;
     const int n = (int)(nc / C), c = (int)(nc % C);
-    const float v = src[((long long)n * Cs + s0 + c) * HW + pix];
-    float* d = dst + ((long long)n * Cd + d0 + c) * HW + pix;
-    if (accumulate) *d += v; else *d = v;
-}
-// residual output out = in + z; MSE loss gradient g = 2 (out - t) / count
-__global__ void residual_mse(const float* in, const float* z, const float* t, float* out, float* g, long long n,
-                             float scale) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float o = in[i] + z[i];
-    out[i] = o;
-    if (g) g[i] = scale * (o - t[i]);
+    dst[((long long)n * Cd + d0 + c) * HW + pix] = src[((long long)n * Cs + s0 + c) * HW + pix];
 }
 __global__ void channel_mean(const float* x, float* y, int C, long long HW, long long n) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -868,12 +863,17 @@ __global__ void channel_mean(const float* x, float* y, int C, long long HW, long
     for (int c = 0; c < C; ++c) s += q[c * HW];
     y[i] = s * (1.0f / (float)C);
 }
-// per-block partial sums of (a - b)^2 in FP64 (fixed order: deterministic loss)
-__global__ __launch_bounds__(256) void sq_diff(const float* a, const float* b, long long n, double* partial) {
+// residual output o = in + z, MSE loss gradient g = 2 (o - t) / count (scale =
+// 2 / count), and per-block partial sums of (o - t)^2 in FP64 (fixed order:
+// deterministic loss)
+__global__ __launch_bounds__(256) void residual_loss(const float* in, const float* z, const float* t, float* g,
+                                                     long long n, float scale, double* partial) {
     __shared__ double red[256];
     double s = 0.0;
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
-        const double d = (double)a[i] - (double)b[i];
+        const float o = in[i] + z[i], ti = t[i];
+        g[i] = scale * (o - ti);
+        const double d = (double)o - (double)ti;
         s += d * d;
     }
     red[threadIdx.x] = s;
@@ -883,6 +883,12 @@ __global__ __launch_bounds__(256) void sq_diff(const float* a, const float* b, l
         __syncthreads();
     }
     if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
+}
+// clears a (na floats) and b (nb of four, 16-byte aligned)
+__global__ __launch_bounds__(256) void clear_two(float* a, long long na, float4* b, long long nb) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i < nb) b[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    else if (i < nb + na) a[i - nb] = 0.f;
 }
 // Adam (Kingma & Ba 2015), bias-corrected
 __global__ void adam_step(float* w, const float* gw, float* m, float* v, long long n, float lr, float b1, float b2,
@@ -910,18 +916,14 @@ hipError_t launch_upsample_fwd(const float* x, float* y, int N, int C, int H, in
     hipLaunchKernelGGL(upsample2_fwd, MSX_GRID((long long)N * C * 4 * H * W), x, y, N, C, H, W, Ct, c0);
     return hipGetLastError();
 }
-hipError_t launch_upsample_bwd(const float* gy, float* gx, int N, int C, int H, int W, int Ct, int c0, hipStream_t s) {
-    hipLaunchKernelGGL(upsample2_bwd, MSX_GRID((long long)N * C * H * W), gy, gx, N, C, H, W, Ct, c0);
+hipError_t launch_cat_bwd(const float* g, float* gup, int C1, float* gskip, int C2, int N, int H, int W,
+                          hipStream_t s) {
+    hipLaunchKernelGGL(cat_bwd, MSX_GRID((long long)N * (C1 + 4LL * C2) * H * W), g, gup, C1, gskip, C2, N, H, W);
     return hipGetLastError();
 }
 hipError_t launch_copy_channels(const float* src, int Cs, int s0, float* dst, int Cd, int d0, int N, int C, int HW,
-                                int accumulate, hipStream_t s) {
-    hipLaunchKernelGGL(copy_channels, MSX_GRID((long long)N * C * HW), src, Cs, s0, dst, Cd, d0, N, C, HW, accumulate);
-    return hipGetLastError();
-}
-hipError_t launch_residual_mse(const float* in, const float* z, const float* t, float* out, float* g, long long n,
-                               float scale, hipStream_t s) {
-    hipLaunchKernelGGL(residual_mse, MSX_GRID(n), in, z, t, out, g, n, scale);
+                                hipStream_t s) {
+    hipLaunchKernelGGL(copy_channels, MSX_GRID((long long)N * C * HW), src, Cs, s0, dst, Cd, d0, N, C, HW);
     return hipGetLastError();
 }
 hipError_t launch_channel_mean(const float* x, float* y, int N, int C, long long HW, hipStream_t s) {
@@ -929,8 +931,13 @@ hipError_t launch_channel_mean(const float* x, float* y, int N, int C, long long
     hipLaunchKernelGGL(channel_mean, MSX_GRID(n), x, y, C, HW, n);
     return hipGetLastError();
 }
-hipError_t launch_sq_diff(const float* a, const float* b, long long n, double* partial, int nblocks, hipStream_t s) {
-    hipLaunchKernelGGL(sq_diff, dim3(nblocks), dim3(256), 0, s, a, b, n, partial);
+hipError_t launch_residual_loss(const float* in, const float* z, const float* t, float* g, long long n, float scale,
+                                double* partial, int nblocks, hipStream_t s) {
+    hipLaunchKernelGGL(residual_loss, dim3(nblocks), dim3(256), 0, s, in, z, t, g, n, scale, partial);
+    return hipGetLastError();
+}
+hipError_t launch_clear(float* a, long long na, float* b, long long nb, hipStream_t s) {
+    hipLaunchKernelGGL(clear_two, MSX_GRID(nb / 4 + na), a, na, reinterpret_cast<float4*>(b), nb / 4);
     return hipGetLastError();
 }
 hipError_t launch_adam(float* w, const float* gw, float* m, float* v, long long n, float lr, float b1, float b2,
