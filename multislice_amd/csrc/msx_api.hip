@@ -1544,6 +1544,28 @@ int multislice_noalloc_impl(msx_ctx ctx, const msx_stack* st, const void* trans,
     return MSX_OK;
 }
 
+// Waves per batch of a STEM scan that chooses none.  Up to 512^2 with lengths
+// that are powers of two the sweeps run at the rate of the last-level cache as
+// long as the part of the waves that they touch (the band, about two thirds)
+// stays in it, so a batch is at most 320 MiB, and batches are equal but for rounding
+// up to 16 waves: a short last one leaves the GPU idle, and launches of odd
+// counts end unevenly (500 FP64 probes of 256 x 512: 125 waves 10366, 128 9375).
+// Whole scans, us, 256 waves at most / this: 64^2 x 3000 probes 3950 / 1764; 128^2
+// x 3000 5959 / 5440; 256^2 x 300 4303 / 3775, x 777 10025 / 8958, x 2000 12595 /
+// 11055 (of 640 waves 12838); 512^2 x 200 5481 / 5279, x 320 8897 / 7768, x 777
+// 16957 / 14550; FP64 512^2 x 200 8756 / 8024, 256^2 x 777 9131 / 9060.  The
+// sweeps of other lengths are bound by arithmetic or latency and want full
+// launches: 384^2 x 500 9694 / 9972, 768^2 x 200 9504 / 10085, 1024^2 x 200 10696
+// / 10578, 2048^2 x 40 8827 / 9282; they keep 256 waves, bounded by 2 GiB.
+template <typename C> int default_batch(int nx, int ny, int nprobe) {
+    const long long bytes = (long long)sizeof(C) * nx * ny;
+    auto pow2 = [](int n) { return (n & (n - 1)) == 0 && n <= 512; };
+    if (!pow2(nx) || !pow2(ny)) return (int)std::max(1LL, std::min<long long>((2LL << 30) / bytes, 256));
+    const int most = (int)std::min<long long>((320LL << 20) / bytes, 1536);
+    const int n = std::max(1, (nprobe + most - 1) / most);
+    return std::min(most, ((nprobe + n - 1) / n + 15) / 16 * 16);
+}
+
 template <typename C>
 int stem_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_probe* pr, const double* pos,
               int nprobe, const msx_detector* det, int ndet, const int32_t* ck, int nck, double weight,
@@ -1553,11 +1575,7 @@ int stem_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_pro
     const long long img = (long long)nx * ny;
     const msx_tuning* tu = ctx->tuning(nx, ny, sizeof(Re) == 8 ? MSX_F64 : MSX_F32);
     if (batch <= 0 && tu && tu->batch > 0) batch = tu->batch;
-    if (batch <= 0) {
-        // default: enough waves to fill the GPU, bounded by ~2 GiB of waves
-        long long b = (2LL << 30) / (long long)(sizeof(C) * img);
-        batch = (int)std::max(1LL, std::min<long long>(b, 256));
-    }
+    if (batch <= 0) batch = default_batch<C>(nx, ny, nprobe);
     batch = std::min(batch, nprobe);
     const C* t_dev = static_cast<const C*>(trans);
     if (where == MSX_HOST) {
