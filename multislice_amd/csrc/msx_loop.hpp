@@ -81,13 +81,6 @@ template <typename C, int NX, int NY> struct LoopShape {
     static constexpr int row_units = NX / LPW;  // work-groups a row phase can use
 };
 
-// a pointer that is the same in every lane, in scalar registers
-template <typename P> __device__ __forceinline__ P* uniform_ptr(P* q) {
-    const unsigned long long v = (unsigned long long)q;
-    return reinterpret_cast<P*>(((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(v >> 32)) << 32) |
-                                (unsigned)__builtin_amdgcn_readfirstlane((unsigned)v));
-}
-
 template <typename C, int NX, int NY>
 __global__ __launch_bounds__((LoopShape<C, NX, NY>::BT)) void slice_loop_kernel(LoopArgs<C> p) {
     using Re = typename real_of<C>::type;

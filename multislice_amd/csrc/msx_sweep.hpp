@@ -109,6 +109,13 @@ __device__ __forceinline__ void sincos_small(float x, float* sn, float* cs) {
     *cs = __uint_as_float(__float_as_uint((k & 1) ? s : c) ^ (((k + 1) & 2) << 30));
 }
 
+// a pointer that is the same in every lane, in scalar registers
+template <typename P> __device__ __forceinline__ P* uniform_ptr(P* q) {
+    const unsigned long long v = (unsigned long long)q;
+    return reinterpret_cast<P*>(((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(v >> 32)) << 32) |
+                                (unsigned)__builtin_amdgcn_readfirstlane((unsigned)v));
+}
+
 // ----------------------------------------------------------------------------
 // Row sweep: lines along the contiguous axis (length N = ny).
 // ----------------------------------------------------------------------------
@@ -117,6 +124,10 @@ template <typename C> struct RowArgs {
     C* psi;                 // out (and in, unless src is set): [nb][nx][N]
     const C* src;           // optional input instead of psi
     long long src_bstride;  // elements between waves of src (0: one input shared by all waves)
+    // per-wave input of a sweep without inverse transform (wave b: src_tab[b])
+    // and output of one without forward transform, instead of psi, or nullptr
+    const C* const* src_tab;
+    C* const* out_tab;
     const C* tw;            // twiddles of length N
     const C* trans;         // transmission [nx][N] shared by all waves, or nullptr
     const C* const* trans_tab;  // per-wave transmission [nx][N] (wave b: trans_tab[b]), or nullptr
@@ -246,6 +257,9 @@ __global__ __launch_bounds__((RowPlanSel<N, PV>::type::T * LPW)) void row_sweep(
             // branch-induced waits)
             const C* img = p.src ? p.src + (long long)__builtin_amdgcn_readfirstlane(b) * p.src_bstride
                                  : p.psi + (long long)__builtin_amdgcn_readfirstlane(b) * p.nx * N;
+            if constexpr (IN == 0 && OUT != 0) {
+                if (p.src_tab) img = uniform_ptr(p.src_tab[b]);
+            }
             const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
                 const_cast<C*>(img), 0, valid ? p.nx * N * (int)sizeof(C) : 0, kBufWord3);
 #pragma unroll
@@ -339,6 +353,9 @@ __global__ __launch_bounds__((RowPlanSel<N, PV>::type::T * LPW)) void row_sweep(
             // and a sweep that stores nothing aim past the bound (dropped):
             // no branch, so no later wait has to count them conservatively
             C* img = p.psi + (long long)__builtin_amdgcn_readfirstlane(b) * p.nx * N;
+            if constexpr (IN != 0 && OUT == 0 && !INTEN) {
+                if (p.out_tab) img = uniform_ptr(p.out_tab[b]);
+            }
             const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
                 img, 0, p.nostore ? 0 : p.nx * N * (int)sizeof(C), kBufWord3);
 #pragma unroll
