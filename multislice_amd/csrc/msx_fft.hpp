@@ -319,14 +319,39 @@ template <> struct RowPlanSel<2048, 1> {
 };
 
 // ---------------------------------------------------------------- LDS views
-// Element m of the line owned by this thread, in LDS.
-//  Contiguous lines: line-major, one padding slot every 16 elements.
-//  Strided lines   : element-major with the WG's lines adjacent (+1 pad per row).
-template <typename C> struct LdsView {
+// Element m of the line owned by this thread, in LDS, at (m + (m >> S)) M: one
+// slot (of M adjacent lines, for the lines of a column tile) inserted after every
+// 2^S elements.  An exchange writes elements R apart and reads consecutive ones,
+// 32 lanes of 8 bytes at a time over 64 banks.
+//  Rows: one slot after every 16 elements.  Others with fewer conflicts in a
+//  model of 32 separate lanes (3 slots after 32: 2.0 -> 1.25 cycles per access
+//  at 512) gained nothing, since the compiler pairs the accesses; the constant
+//  parts of the addresses as instruction offsets did (512 FP32: 8 address
+//  registers and their arithmetic less; 320 probes of 512^2 x 100 slices 34.55
+//  -> 34.2 ms).
+//  Column tiles: a slot (TW elements) after every 2^S, S from the first radix,
+//  where one element after every TW was 1.5 to 2.5 cycles per access (256: 1.5,
+//  512: 1.75, 1024: 2.0, 2048: 2.5; counters agree) and is 1.0 now, 1.1-1.2 at
+//  384 and 768.  FP32 slice sweeps, us: 2048^2 x 8 waves 145 -> 130, 1024^2 x 40
+//  140 -> 125.  Whole calls of 16 slices: 3 waves of 2048^2 2172 -> 1934, 12 of
+//  768^2 1302 -> 1244, 6 of 1024^2 1158 -> 1108, 60 of 384^2 1390 -> 1376.
+template <typename C, int S, int M> struct LdsView {
     C* base;
-    int stride;  // distance between consecutive elements (in C units)
-    bool padded;
-    __device__ __forceinline__ C* at(int m) const { return base + (padded ? (m + (m >> 4)) : m * stride); }
+    static __device__ __forceinline__ constexpr int off(int m) { return (m + (m >> S)) * M; }
+    // element v + c; DISJOINT: v and c have no bit in common, so that the
+    // constant part stays out of the address arithmetic
+    template <bool DISJOINT> __device__ __forceinline__ C* at(int v, int c) const {
+        return DISJOINT ? base + off(v) + off(c) : base + off(v + c);
+    }
+};
+template <class PL, typename C> struct RowLds {
+    static constexpr int len = PL::N + (PL::N >> 4);
+    using View = LdsView<C, 4, 1>;
+};
+template <class PL, typename C, int TW> struct ColLds {
+    static constexpr int S = PL::R[0] == 6 || PL::R[0] >= 16 ? 4 : 3;  // 384: 4 is 1.5-2% faster than 3
+    static constexpr int len = (PL::N + (PL::N >> S)) * TW;
+    using View = LdsView<C, S, TW>;
 };
 
 // ---------------------------------------------------------------- twiddles
@@ -399,11 +424,12 @@ template <bool WAVE> __device__ __forceinline__ void lds_sync() {
 // DB (double buffering): exchange x of a line uses LDS buffer x & 1, so the
 // write of exchange x+1 cannot overtake reads of exchange x and one barrier
 // per exchange suffices; X is the running exchange index.
-template <int N, int T, int R, int Ns, int S, bool LAST, bool WAVE, bool DB, int X, int TWOFF, typename C>
-__device__ __forceinline__ void stockham_pass(C (&a)[N / T], int t, const LdsView<C> (&lds)[2], const C* w) {
+template <int N, int T, int R, int Ns, int S, bool LAST, bool WAVE, bool DB, int X, int TWOFF, typename C, class L>
+__device__ __forceinline__ void stockham_pass(C (&a)[N / T], int t, const L (&lds)[2], const C* w) {
     constexpr int Q = N / (R * T);
     static_assert(Q * R * T == N, "radix/thread split must tile N");
-    const LdsView<C>& L = lds[DB ? (X & 1) : 0];
+    const L& line = lds[DB ? (X & 1) : 0];
+    constexpr auto pow2 = [](int n) { return (n & (n - 1)) == 0; };
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         C b[R];
@@ -425,19 +451,19 @@ __device__ __forceinline__ void stockham_pass(C (&a)[N / T], int t, const LdsVie
         } else {
             const int base = (j / Ns) * Ns * R + (j % Ns);
 #pragma unroll
-            for (int r = 0; r < R; ++r) *L.at(base + r * Ns) = b[r];
+            for (int r = 0; r < R; ++r) *line.template at<pow2(R) && pow2(Ns)>(base, r * Ns) = b[r];
         }
     }
     if constexpr (!LAST) {
         lds_sync<WAVE>();
 #pragma unroll
-        for (int e = 0; e < N / T; ++e) a[e] = *L.at(t + e * T);
+        for (int e = 0; e < N / T; ++e) a[e] = *line.template at<pow2(T)>(t, e * T);
         if constexpr (!DB) lds_sync<WAVE>();
     }
 }
 
-template <class PL, int I, int Ns, int S, bool WAVE, bool DB, int X, typename C>
-__device__ __forceinline__ void run_passes(C (&a)[PL::N / PL::T], int t, const LdsView<C> (&lds)[2], const C* w) {
+template <class PL, int I, int Ns, int S, bool WAVE, bool DB, int X, typename C, class L>
+__device__ __forceinline__ void run_passes(C (&a)[PL::N / PL::T], int t, const L (&lds)[2], const C* w) {
     if constexpr (I < PL::P) {
         constexpr int R = PL::R[I];
         constexpr bool LAST = I == PL::P - 1;
@@ -449,9 +475,8 @@ __device__ __forceinline__ void run_passes(C (&a)[PL::N / PL::T], int t, const L
 // Full length-N transform of the registers a[] (unscaled), sign S.  With DB,
 // X0 is the index of the transform's first exchange; a transform performs
 // PL::P - 1 exchanges.
-template <class PL, int S, bool WAVE, bool DB = false, int X0 = 0, typename C>
-__device__ __forceinline__ void fft_line(C (&a)[PL::N / PL::T], int t, const LdsView<C> (&lds)[2],
-                                         const TwReg<PL, C>& tw) {
+template <class PL, int S, bool WAVE, bool DB = false, int X0 = 0, typename C, class L>
+__device__ __forceinline__ void fft_line(C (&a)[PL::N / PL::T], int t, const L (&lds)[2], const TwReg<PL, C>& tw) {
     run_passes<PL, 0, 1, S, WAVE, DB, X0>(a, t, lds, tw.w);
 }
 

@@ -30,7 +30,7 @@ static_assert(!kColAlt || kTc<1> == kTc<0>, "column plan variants share the thre
 template <int PV> constexpr int row_lpw() { return kT<PV> >= 256 ? 1 : 256 / kT<PV>; }
 
 // columns per work-group of the column sweep (coalescing width), bounded by
-// 1024 threads and by the LDS tile N*(TW+1) complex values
+// 1024 threads and by an LDS tile of N*(TW+1) complex values
 #ifndef MSX_COL_TW
 #define MSX_COL_TW 16
 #endif
@@ -86,7 +86,7 @@ hipError_t row_go(const RowArgs<C>& a0, hipStream_t s) {
     a.wpb = pick_wpb(a.wpb, (long long)nxg * a.nb, 4096);
     const long long nchunk = (a.nb + a.wpb - 1) / a.wpb;
     const unsigned grid = (unsigned)(nxg * nchunk);
-    const size_t smem = (size_t)LPW * (kN + kN / 16) * sizeof(C);
+    constexpr size_t smem = LPW * RowLds<typename RowPlanSel<kN, PV>::type, C>::len * sizeof(C);
     auto k = row_sweep<C, kN, IN, OUT, LPW, VREAL, INTEN, PV>;
     hipError_t e = set_smem(k, smem);
     if (e != hipSuccess) return e;
@@ -124,12 +124,13 @@ template <typename C, int IN, int OUT, int OPS, int TW, int PV>
 hipError_t col_go_tw(const ColArgs<C>& a0, hipStream_t s) {
     ColArgs<C> a = a0;
     const int groups = (a.ny + TW - 1) / TW;
-    constexpr size_t tile = (size_t)kN * (TW + 1) * sizeof(C);
+    using PL = typename ColPlanSel<kN, PV>::type;
+    constexpr size_t tile = ColLds<PL, C, TW>::len * sizeof(C);
     // double-buffer the exchanges when two tiles fit in the work-group LDS
     // limit (a launch asking for the full 160 KiB is refused)
     constexpr bool DB = MSX_COL_DB && 2 * tile <= 150 * 1024;
     auto k = col_sweep<C, kN, IN, OUT, TW, OPS, DB, PV>;
-    constexpr size_t smem = col_lds_bytes<C, kN, TW, DB>();
+    constexpr size_t smem = col_lds_bytes<PL, C, TW, DB>();
     hipError_t e = set_smem(k, smem);
     if (e != hipSuccess) return e;
     unsigned grid;

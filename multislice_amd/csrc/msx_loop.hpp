@@ -75,7 +75,9 @@ template <typename C, int NX, int NY> struct LoopShape {
     // 0.98 -> 1.22x); FP64 tiles of 4 are as wide, and 512 threads spill
     static constexpr int BT = sizeof(C) == 8 && 8 * PC::T > 256 ? 8 * PC::T : 256;
     static constexpr int LPW = BT / PR::T, TW = BT / PC::T;
-    static constexpr size_t tile = (size_t)NX * (TW + 1) * sizeof(C), row = (size_t)LPW * (NY + NY / 16) * sizeof(C);
+    using LR = RowLds<PR, C>;
+    using LC = ColLds<PC, C, TW>;
+    static constexpr size_t tile = LC::len * sizeof(C), row = LPW * LR::len * sizeof(C);
     static constexpr bool DB = 2 * tile <= 75 * 1024;  // two work-groups per CU
     static constexpr size_t lds = row > (DB ? 2 : 1) * tile ? row : (DB ? 2 : 1) * tile;
     static constexpr int row_units = NX / LPW;  // work-groups a row phase can use
@@ -99,7 +101,8 @@ __global__ __launch_bounds__((LoopShape<C, NX, NY>::BT)) void slice_loop_kernel(
 
     // row phase: line lw, position t
     const int lw = tid / T, t = tid % T;
-    const LdsView<C> rlds[2] = {{smem + lw * (NY + NY / 16), 1, true}, {smem + lw * (NY + NY / 16), 1, true}};
+    using LR = typename S::LR;
+    const typename LR::View rlds[2] = {{smem + lw * LR::len}, {smem + lw * LR::len}};
     TwReg<PR, C> twr;
     load_twiddles<PR>(twr, t, p.twy);
     unsigned inb = 0;
@@ -107,7 +110,8 @@ __global__ __launch_bounds__((LoopShape<C, NX, NY>::BT)) void slice_loop_kernel(
     for (int e = 0; e < E; ++e) inb |= (t + e * T < p.blo || t + e * T >= NY - p.bhi ? 1u : 0u) << e;
     // column phase: column cw of a tile, position tc
     const int cw = tid % TW, tc = tid / TW;
-    const LdsView<C> clds[2] = {{smem + cw, TW + 1, false}, {smem + NX * (TW + 1) + cw, TW + 1, false}};
+    using LC = typename S::LC;
+    const typename LC::View clds[2] = {{smem + cw}, {smem + LC::len + cw}};
     TwReg<PC, C> twc;
     load_twiddles<PC>(twc, tc, p.twx);
     float kx2[Ec];

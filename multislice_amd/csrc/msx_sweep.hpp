@@ -176,7 +176,8 @@ __global__ __launch_bounds__((RowPlanSel<N, PV>::type::T * LPW)) void row_sweep(
     const bool live = ix_raw < p.nx;
     const int ix = live ? ix_raw : p.nx - 1;  // dead rows compute, never store
     const int b0 = chunk * p.wpb, b1 = min(p.nb, b0 + p.wpb);
-    const LdsView<C> lds[2] = {{smem + lw * (N + N / 16), 1, true}, {smem + lw * (N + N / 16), 1, true}};
+    using LV = RowLds<PL, C>;
+    const typename LV::View lds[2] = {{smem + lw * LV::len}, {smem + lw * LV::len}};
     // element offset of (this line, y) in a wave's image
     auto eo = [&](int y) -> unsigned { return (unsigned)ix * (unsigned)N + (unsigned)y; };
 
@@ -485,8 +486,8 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblk) {
 }
 // Bytes of the column sweep's dynamic LDS: the exchange buffers, which also
 // hold the detector reduction scratch (at least 2 KiB).
-template <typename C, int N, int TW, bool DB> constexpr size_t col_lds_bytes() {
-    constexpr size_t tile = (size_t)N * (TW + 1) * sizeof(C);
+template <class PL, typename C, int TW, bool DB> constexpr size_t col_lds_bytes() {
+    constexpr size_t tile = ColLds<PL, C, TW>::len * sizeof(C);
     constexpr size_t x = DB ? 2 * tile : tile;
     return x < 2048 ? 2048 : x;
 }
@@ -606,7 +607,8 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
         b = b0 + i;
         return b < b1;
     };
-    const LdsView<C> lds[2] = {{smem + lw, TW + 1, false}, {smem + N * (TW + 1) + lw, TW + 1, false}};
+    using LV = ColLds<PL, C, TW>;
+    const typename LV::View lds[2] = {{smem + lw}, {smem + LV::len + lw}};
     constexpr bool gen = (OPS & kColGen) != 0;
     constexpr bool point = (OPS & (kColProp | kColMask | kColDetect | kColCtf)) != 0;
 
