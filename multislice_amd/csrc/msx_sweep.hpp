@@ -147,8 +147,13 @@ template <typename C> struct RowArgs {
     int prune;
     // with inten set: iacc 0 writes |psi|^2, 1 writes iw*|psi|^2, 2 adds
     // iw*|psi|^2 to what inten holds (weighted sums over several launches)
+    // with isteps > 1 the waves are images of nb / isteps waves at isteps steps
+    // each (image b: wave b / isteps, step b % isteps, weight iws[step]), wpb =
+    // isteps, and inten holds one sum per wave
     int iacc;
     Re iw;
+    int isteps;
+    const Re* iws;
     int nostore;  // 1: only the intensity is written, not the wave
     int plan;  // FFT plan variant (RowPlanSel)
 };
@@ -287,10 +292,12 @@ __global__ __launch_bounds__((RowPlanSel<N, PV>::type::T * LPW)) void row_sweep(
     if (MSX_ROW_DRAIN) __builtin_amdgcn_s_waitcnt(0);
     // |psi|^2 output of wave b: [nb][nx][N] reals
     auto inten_rsrc = [&](int b) {
-        return __builtin_amdgcn_make_buffer_rsrc(p.inten + (long long)__builtin_amdgcn_readfirstlane(b) * p.nx * N, 0,
+        const int w = __builtin_amdgcn_readfirstlane(p.isteps > 1 ? b / p.isteps : b);
+        return __builtin_amdgcn_make_buffer_rsrc(p.inten + (long long)w * p.nx * N, 0,
                                                  p.nx * N * (int)sizeof(Re), kBufWord3);
     };
     const unsigned row0 = (unsigned)ix * (unsigned)N;
+    Re oi[INTEN ? E : 1];
     // one wave: its row is in cur (with the prefetch) or loaded here; the
     // next wave's row is prefetched into next
     auto wave = [&](int b, C (&cur)[E], C (&next)[E]) {
@@ -316,10 +323,10 @@ __global__ __launch_bounds__((RowPlanSel<N, PV>::type::T * LPW)) void row_sweep(
         } else {
             load(b, cur);
         }
-        Re oi[INTEN ? E : 1];
+        const bool first = p.isteps <= 1 || b == b0, last = p.isteps <= 1 || b + 1 == b1;
         if constexpr (INTEN) {
             // the running sums this wave adds to, loaded with its row
-            if (p.iacc == 2) {
+            if (p.iacc == 2 && first) {
 #pragma unroll
                 for (int e = 0; e < E; ++e)
                     oi[e] = buf_load<Re>(inten_rsrc(b), (row0 + (unsigned)(t + e * T)) * (unsigned)sizeof(Re));
@@ -340,12 +347,14 @@ __global__ __launch_bounds__((RowPlanSel<N, PV>::type::T * LPW)) void row_sweep(
         if constexpr (INTEN) {
             // buffer stores (dead rows aim past the bound)
             const __amdgpu_buffer_rsrc_t ri = inten_rsrc(b);
+            const Re iw = p.isteps > 1 ? p.iws[b - b0] : p.iw;
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 Re v = cnorm2(cur[e]);
-                if (p.iacc != 0) v = p.iw * v;
-                if (p.iacc == 2) v = oi[e] + v;
-                buf_store(v, ri, live ? (row0 + (unsigned)(t + e * T)) * (unsigned)sizeof(Re) : kBufDrop);
+                if (p.iacc != 0) v = iw * v;
+                if (p.iacc == 2 || !first) v = oi[e] + v;
+                oi[e] = v;
+                buf_store(v, ri, live && last ? (row0 + (unsigned)(t + e * T)) * (unsigned)sizeof(Re) : kBufDrop);
             }
         }
         if constexpr (OUT != 0) fft_line<PL, OUT, WAVE>(cur, t, lds, tw);
@@ -419,6 +428,10 @@ template <typename C> struct ColArgs {
     double a2, phi2, a3, phi3;
     int astig;
     C* out;                // store target (nullptr: in place)
+    // kColCtf with steps > 0: output b is wave b / steps at the defocus
+    // dfs[b % steps] (out set; nb counts outputs)
+    const double* dfs;
+    int steps;
     int ny, nb, ops;
     int wpb;               // > 0: waves per work-group (chunked); < 0: balanced schedule (below)
     int tile;              // columns per work-group (0: the built-in width for this length)
@@ -654,7 +667,8 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
     const int img_bytes = N * p.ny * (int)sizeof(C);
     auto load = [&](int g, int b, bool valid, C (&v)[E]) {
         const int ld_col = live_col(g * TW + lw) ? lw : first_live(g);
-        const C* img = p.psi + (long long)__builtin_amdgcn_readfirstlane(b) * N * p.ny;
+        const int w = (OPS & kColCtf) != 0 && p.steps > 1 ? b / p.steps : b;
+        const C* img = p.psi + (long long)__builtin_amdgcn_readfirstlane(w) * N * p.ny;
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<C*>(img), 0,
                                                                              valid ? img_bytes : 0, kBufWord3);
         const unsigned off0 = elem(g * TW + ld_col) * (unsigned)sizeof(C);
@@ -716,6 +730,7 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
         const int iy = col_y(g);
         const bool live = live_col(g * TW + lw);
         const double ky = (gen || (OPS & kColCtf)) ? (double)freq_index(iy, p.ny) / p.by : 0.0;
+        const double df = (OPS & kColCtf) != 0 && p.steps > 0 ? p.dfs[b % p.steps] : p.df;
         const double oy = (OPS & kColObl) ? (double)freq_index(iy, p.ny) / p.obl_bsg : 0.0;
         if constexpr (gen) {
             const double2 pos = p.pos[b];
@@ -765,7 +780,7 @@ __global__ __launch_bounds__((ColPlanSel<N, PV>::type::T * TW), MSX_COL_MINW) vo
                     if (k2 <= p.kap_hi) {
                         const double kx = (double)freq_index(t + e * T, N) / p.ax;
                         const double kk = kx * kx + ky * ky;
-                        double w = p.chi2 * kk - p.df;
+                        double w = p.chi2 * kk - df;
                         if (p.astig) {
                             // mulslice.cpp:620-628
                             const double phi = atan2(ky, kx);
