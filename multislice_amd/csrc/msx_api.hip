@@ -838,11 +838,12 @@ template <typename C> void loop_tables(const SliceTables<C>& tb, LoopArgs<C>* a)
     a->blo = tb.band.lo, a->bhi = tb.band.hi;
 }
 
-// slices [s0, s1) of nb waves in one kernel; real_in and mixed_out as in
-// slice_loop_body
+// slices [s0, s1) of nb waves in one kernel; start and mixed_out as in
+// slice_loop_body (with start 1 the waves of slice 0 may fill columns outside
+// the band: a probe's aperture can be wider)
 template <typename C>
 int persistent_loop(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, const C* trans, C* psi, int nb,
-                    const C* src, long long src_bstride, int s0, int s1, bool real_in, bool mixed_out, bool* done) {
+                    const C* src, long long src_bstride, int s0, int s1, int start, bool mixed_out, bool* done) {
     *done = false;
     if (is_oblique(st) || !loop_wanted<C>(ctx, st->nx, st->ny, nb, s1 - s0)) return MSX_OK;
     LoopArgs<C> a;
@@ -870,7 +871,8 @@ int persistent_loop(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, 
     a.s0 = s0;
     a.s1 = s1;
     a.nb = nb;
-    a.first_real = real_in;
+    a.first_real = s0 == 0 && start == 0;
+    a.first_all = s0 == 0;
     a.mixed = mixed_out;
     return loop_go<C>(ctx, st->nx, st->ny, a, 2u * (unsigned)(s1 - s0), done);
 }
@@ -892,8 +894,7 @@ int slice_loop(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, const
                const C* src, long long src_bstride, int start, DetPlan* det, bool mixed_out = false) {
     if (!ctx->graphs && !det) {
         bool done = false;
-        CHK(persistent_loop<C>(ctx, st, tb, trans, psi, nb, src, src_bstride, 0, st->nslice, start == 0, mixed_out,
-                               &done));
+        CHK(persistent_loop<C>(ctx, st, tb, trans, psi, nb, src, src_bstride, 0, st->nslice, start, mixed_out, &done));
         if (done) return MSX_OK;
     } else if (!ctx->graphs) {
         // up to each checkpoint's slice, whose column sweep sums the detectors
@@ -901,8 +902,7 @@ int slice_loop(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, const
         for (int k = 0; k < det->nck; k++) {
             const int c = det->ck[k];
             bool done = false;
-            CHK(persistent_loop<C>(ctx, st, tb, trans, psi, nb, src, src_bstride, s, c - 1, s == 0 && start == 0, true,
-                                   &done));
+            CHK(persistent_loop<C>(ctx, st, tb, trans, psi, nb, src, src_bstride, s, c - 1, start, true, &done));
             CHK(slice_loop_body<C>(ctx, st, tb, trans, psi, nb, src, src_bstride, start, det, mixed_out, nullptr,
                                    done ? c - 1 : s, c));
             s = c;
@@ -1200,7 +1200,7 @@ int batch_class(msx_ctx ctx, const msx_job* jobs, std::vector<BatchItem>& g, std
         a.trans_tab = dtt;
         a.prop_tab = dpt;
         a.nb = nb;
-        a.first_real = 1;
+        a.first_real = a.first_all = 1;
         bool done = false;
         CHK(loop_go<C>(ctx, nx, ny, a, 2u * (unsigned)S, &done));
         if (done) {
