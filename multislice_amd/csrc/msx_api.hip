@@ -1288,14 +1288,7 @@ int check_stack(const msx_stack* st);
 template <typename C> bool jobs_apart(msx_ctx ctx, const msx_job* jobs, int njobs) {
     typedef std::pair<uintptr_t, uintptr_t> Range;  // [first, second)
     std::vector<Range> out(njobs);
-    auto own = [&](const void* q) {
-        hipPointerAttribute_t at;
-        if (hipPointerGetAttributes(&at, q) != hipSuccess) {
-            (void)hipGetLastError();
-            return false;
-        }
-        return at.type == hipMemoryTypeDevice && at.device == ctx->device && (uintptr_t)q % sizeof(C) == 0;
-    };
+    auto own = [&](const void* q) { return msx_ctx_owns(ctx, q, sizeof(C)); };
     for (int i = 0; i < njobs; i++) {
         const msx_job& j = jobs[i];
         if (!own(j.psi) || (j.psi0 && !own(j.psi0))) return false;
@@ -2386,6 +2379,14 @@ int potential_rs_impl(msx_ctx ctx, const msx_atom* atoms, int64_t natoms, const 
 
 int msx_ctx_device(const msx_ctx_s* ctx) { return ctx->device; }
 hipStream_t msx_ctx_stream(const msx_ctx_s* ctx) { return ctx->stream; }
+bool msx_ctx_owns(const msx_ctx_s* ctx, const void* q, size_t align) {
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, q) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice && at.device == ctx->device && (uintptr_t)q % align == 0;
+}
 int msx_ctx_scratch(msx_ctx_s* ctx, size_t bytes, void** out) {
     CHK(ctx->unitbuf.ensure(bytes));
     *out = ctx->unitbuf.p;

@@ -318,6 +318,9 @@ int fail(int code, const char* fmt, ...);
 struct msx_ctx_s;
 int msx_ctx_device(const msx_ctx_s* ctx);
 hipStream_t msx_ctx_stream(const msx_ctx_s* ctx);
+// whether q is memory of the context's own device, aligned as given: what its
+// kernels may read and write in place
+bool msx_ctx_owns(const msx_ctx_s* ctx, const void* q, size_t align);
 // a device buffer of the context, at least `bytes` long; its contents last
 // until the next call that asks for it
 int msx_ctx_scratch(msx_ctx_s* ctx, size_t bytes, void** out);

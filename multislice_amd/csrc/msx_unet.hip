@@ -403,15 +403,18 @@ int check_shape(msx_unet net, int n, int h, int w, int where) {
     return MSX_OK;
 }
 // the inputs (*x [n][cin0][h][w], optional target *t [n][h][w]) on the GPU:
-// device tensors are read where they are (every call waits for its work),
-// host ones are copied into the workspace
+// tensors of this device are read where they are (every call waits for its
+// work), all others (host buffers, another device's or pinned memory, whose
+// addresses this device's kernels may not reach) are copied into the workspace
 int stage_inputs(msx_unet net, const float** x, const float** t, int where) {
-    if (where == MSX_DEVICE) return MSX_OK;
     const size_t bytes = sizeof(float) * (size_t)net->wn * net->wh * net->ww;
-    UHIP(hipMemcpyAsync(net->xin, *x, bytes * net->cin0, hipMemcpyHostToDevice, net->stream()));
-    *x = net->xin;
-    if (t) {
-        UHIP(hipMemcpyAsync(net->tin, *t, bytes, hipMemcpyHostToDevice, net->stream()));
+    const hipMemcpyKind kind = where == MSX_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
+    if (where == MSX_HOST || !msx_ctx_owns(net->ctx, *x, sizeof(float))) {
+        UHIP(hipMemcpyAsync(net->xin, *x, bytes * net->cin0, kind, net->stream()));
+        *x = net->xin;
+    }
+    if (t && (where == MSX_HOST || !msx_ctx_owns(net->ctx, *t, sizeof(float)))) {
+        UHIP(hipMemcpyAsync(net->tin, *t, bytes, kind, net->stream()));
         *t = net->tin;
     }
     return MSX_OK;
@@ -581,11 +584,11 @@ MSX_API int msx_unet_forward(msx_unet net, const float* x, float* y, int n, int 
     UHIP(hipSetDevice(msx_ctx_device(net->ctx)));
     UCHK(net->workspace(n, h, w));
     UCHK(stage_inputs(net, &x, nullptr, where));
-    // straight into y unless it is a host buffer or shares memory with x
-    // (the head's tiles read x while others write)
+    // straight into y unless it is not this device's memory or shares memory
+    // with x (the head's tiles read x while others write)
     const size_t cnt = (size_t)n * h * w;
     const bool apart = y + cnt <= x || x + cnt * net->cin0 <= y;
-    float* dst = where == MSX_DEVICE && apart ? y : net->out;
+    float* dst = where == MSX_DEVICE && apart && msx_ctx_owns(net->ctx, y, sizeof(float)) ? y : net->out;
     UCHK(net->forward(x, dst));
     if (dst != y)
         UHIP(hipMemcpyAsync(y, dst, sizeof(float) * cnt,
