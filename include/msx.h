@@ -114,6 +114,11 @@ typedef struct msx_tuning {
 MSX_API int msx_autotune(msx_ctx ctx, int nx, int ny, int prec, int max_batch, msx_tuning* best);
 MSX_API int msx_set_tuning(msx_ctx ctx, int nx, int ny, int prec, const msx_tuning* t);
 MSX_API int msx_graph_stats(msx_ctx ctx, int64_t* captures, int64_t* replays);
+/* Without graphs, slice loops of few small waves (lengths 128 to 512) run as
+ * one persistent kernel instead of two launches per slice: how many the
+ * context has launched, and in how many calls one gave up waiting for its
+ * work-groups (either may be NULL). */
+MSX_API int msx_loop_stats(msx_ctx ctx, int64_t* loops, int64_t* given_up);
 
 /* Kernel timing (the reference timed its loops with cudaEvents and printed
  * them, ModelPotential.cu:46-50,92-96 and ModelSimulated.cu:43-47,178-182).

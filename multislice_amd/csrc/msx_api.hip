@@ -237,6 +237,7 @@ struct msx_ctx_s {
     unsigned loop_epoch = 0;
     int* loop_status = nullptr;
     int coop = -1;  // cooperative launches: not asked / no / yes
+    long long loops = 0, loops_given_up = 0;  // persistent loops launched, and calls in which one gave up
     int ensure_pinned(size_t n) {
         if (n <= h_pin_cap) return MSX_OK;
         if (h_pin) HIPCHK(hipHostFree(h_pin));
@@ -822,11 +823,15 @@ template <typename C> int loop_go(msx_ctx ctx, int nx, int ny, LoopArgs<C>& a, u
     a.spin = kLoopSpin;
     a.status = ctx->loop_status;
     ctx->loop_epoch += passes * (unsigned)((a.nb + teams - 1) / teams);
-    // a stream or device that takes no cooperative launch runs the sweeps
-    if (launch_loop<C>(nx, ny, a, teams, ctx->stream) != hipSuccess) {
+    // a device or stream without room for a cooperative launch runs the sweeps
+    const hipError_t e = launch_loop<C>(nx, ny, a, teams, ctx->stream);
+    if (e == hipErrorCooperativeLaunchTooLarge || e == hipErrorNotSupported || e == hipErrorOutOfMemory ||
+        e == hipErrorLaunchOutOfResources) {
         (void)hipGetLastError();
         return MSX_OK;
     }
+    HIPCHK(e);
+    ctx->loops++;
     *done = true;
     return MSX_OK;
 }
@@ -880,6 +885,7 @@ int persistent_loop(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, 
 int loop_failed(msx_ctx ctx) {
     if (!ctx->loop_status || *ctx->loop_status == 0) return MSX_OK;
     *ctx->loop_status = 0;
+    ctx->loops_given_up++;
     ctx->loopbuf.release();  // the next loop starts from cleared flags
     return fail(MSX_EHIP, "slice loop: a barrier between its work-groups gave up");
 }
@@ -2535,6 +2541,13 @@ MSX_API int msx_graph_stats(msx_ctx ctx, int64_t* captures, int64_t* replays) {
     if (!ctx) return fail(MSX_ESTATE, "ctx is NULL");
     if (captures) *captures = ctx->graph_captures;
     if (replays) *replays = ctx->graph_hits;
+    return MSX_OK;
+}
+
+MSX_API int msx_loop_stats(msx_ctx ctx, int64_t* loops, int64_t* given_up) {
+    if (!ctx) return fail(MSX_ESTATE, "ctx is NULL");
+    if (loops) *loops = ctx->loops;
+    if (given_up) *given_up = ctx->loops_given_up;
     return MSX_OK;
 }
 

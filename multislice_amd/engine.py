@@ -87,7 +87,7 @@ class Lens(C.Structure):
 
 PROF_ROW, PROF_COL, PROF_SPLAT, PROF_DET = 0, 1, 2, 3
 
-EXPORTS = ["msx_create", "msx_destroy", "msx_set_stream", "msx_wait_stream", "msx_set_graphs", "msx_graph_stats", "msx_autotune",
+EXPORTS = ["msx_create", "msx_destroy", "msx_set_stream", "msx_wait_stream", "msx_set_graphs", "msx_graph_stats", "msx_loop_stats", "msx_autotune",
            "msx_set_tuning", "msx_last_error", "msx_version",
            "msx_profile", "msx_profile_read", "msx_copy_probe", "msx_displace", "msx_philox4x32_10",
            "msx_wavelength", "msx_sigma", "msx_vzatom", "msx_featom", "msx_fft2d", "msx_potential",
@@ -140,6 +140,7 @@ def load():
         "msx_wait_stream": (i, [vp, vp]),
         "msx_set_graphs": (i, [vp, i]),
         "msx_autotune": (i, [vp, i, i, i, i, C.POINTER(Tuning)]), "msx_set_tuning": (i, [vp, i, i, i, C.POINTER(Tuning)]), "msx_graph_stats": (i, [vp, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
+        "msx_loop_stats": (i, [vp, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
         "msx_last_error": (C.c_char_p, []), "msx_version": (i, []),
         "msx_profile": (i, [vp, i]),
         "msx_profile_read": (i, [vp, i, C.POINTER(C.c_int64), C.POINTER(d), C.POINTER(d)]),
@@ -332,6 +333,12 @@ class Context:
         c, r = C.c_int64(), C.c_int64()
         _check(load().msx_graph_stats(self.h, C.byref(c), C.byref(r)))
         return c.value, r.value
+
+    def loop_stats(self):
+        """(launched, given up) persistent slice loops so far (msx_loop_stats)."""
+        n, g = C.c_int64(), C.c_int64()
+        _check(load().msx_loop_stats(self.h, C.byref(n), C.byref(g)))
+        return n.value, g.value
 
     def profile(self, enable=True):
         """Turn per-kernel event timing on/off (resets the totals)."""

@@ -1,0 +1,69 @@
+"""Which calls the persistent slice loop takes: its launches are counted, so
+that the tests that compare it with the sweeps cannot compare the sweeps with
+themselves."""
+import numpy as np
+import pytest
+
+import multislice_amd as msx
+
+pytestmark = pytest.mark.gpu
+
+KEV = 200.0
+
+
+def trans(n, ns, f64=False):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n)
+    ph = torch.rand((ns, n, n), generator=g, device="cuda", dtype=torch.float64 if f64 else torch.float32)
+    return torch.polar(torch.ones_like(ph), ph)
+
+
+def launched(ctx, fn):
+    n0, bad0 = ctx.loop_stats()
+    fn()
+    n1, bad1 = ctx.loop_stats()
+    assert bad1 == bad0
+    return n1 - n0
+
+
+@pytest.mark.parametrize("f64", [False, True])
+@pytest.mark.parametrize("n,nwave", [(128, 1), (128, 256), (256, 5), (384, 2), (512, 1)])
+def test_exit_waves(ctx, n, nwave, f64):
+    import torch
+    ns, a = 20, 0.1 * n
+    t = trans(n, ns, f64)
+    psi = torch.ones((nwave, n, n), dtype=t.dtype, device="cuda")
+
+    def go(m=ns):
+        ctx.multislice(t, np.full(ns, 2.0), np.arange(m), psi, a, a, KEV)
+    assert launched(ctx, go) == 1
+    assert launched(ctx, lambda: go(2)) == 0  # few slices
+    ctx.set_graphs(True)
+    assert launched(ctx, go) == 0
+    ctx.set_graphs(False)
+    ctx.profile(True)
+    assert launched(ctx, go) == 0
+    ctx.profile(False)
+
+
+def test_lengths_without_a_loop(ctx):
+    import torch
+    for n in (64, 768):
+        t = trans(n, 20)
+        psi = torch.ones((1, n, n), dtype=t.dtype, device="cuda")
+        assert launched(ctx, lambda: ctx.multislice(t, np.full(20, 2.0), np.arange(20), psi, 10.0, 10.0, KEV)) == 0
+
+
+def test_stem_partial_coherence_and_job_sets(ctx):
+    import torch
+    n, ns, a = 128, 20, 12.8
+    t, cz, layer = trans(n, ns), np.full(ns, 2.0), np.arange(ns)
+    pos = np.random.default_rng(0).uniform(0, a, (9, 2))
+    # a loop up to each checkpoint's slice, for each of three batches
+    assert launched(ctx, lambda: ctx.stem(t, cz, layer, a, a, KEV, dict(alpha_max=0.02), pos, [(0, 1.0)], [10, 20],
+                                          batch=3)) == 6
+    lens = dict(cs=1e7, df=500.0, aobj=0.02)
+    assert launched(ctx, lambda: ctx.partial_coherence(t, cz, layer, a, a, KEV, lens, 0.0, 5e-3, 30.0, 15.0)) == 1
+    jobs = [dict(trans=t, psi=torch.ones((n, n), dtype=t.dtype, device="cuda"), ax=a, by=a, kev=KEV, cz=cz,
+                 layer=layer) for _ in range(3)]
+    assert launched(ctx, lambda: ctx.multislice_batch(jobs)) == 1
