@@ -851,6 +851,8 @@ int persistent_loop(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, 
                     const C* src, long long src_bstride, int s0, int s1, int start, bool mixed_out, bool* done) {
     *done = false;
     if (is_oblique(st) || !loop_wanted<C>(ctx, st->nx, st->ny, nb, s1 - s0)) return MSX_OK;
+    // the exchange past the caches is for memory of this device alone
+    if (!msx_ctx_owns(ctx, psi, sizeof(C))) return MSX_OK;
     LoopArgs<C> a;
     std::memset(&a, 0, sizeof a);
     loop_tables(tb, &a);

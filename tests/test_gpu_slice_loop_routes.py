@@ -67,3 +67,19 @@ def test_stem_partial_coherence_and_job_sets(ctx):
     jobs = [dict(trans=t, psi=torch.ones((n, n), dtype=t.dtype, device="cuda"), ax=a, by=a, kev=KEV, cz=cz,
                  layer=layer) for _ in range(3)]
     assert launched(ctx, lambda: ctx.multislice_batch(jobs)) == 1
+
+
+def test_waves_in_pinned_memory(ctx):
+    """The work-groups exchange waves in this device's memory only: others go through the sweeps."""
+    import ctypes as C
+    import torch
+    n, ns, a = 128, 20, 12.8
+    t, cz, layer = trans(n, ns), np.full(ns, 2.0), np.arange(ns)
+    want = torch.ones((1, n, n), dtype=t.dtype, device="cuda")
+    psi = torch.empty(want.shape, dtype=want.dtype, pin_memory=True)
+    psi.copy_(want)
+    ctx.multislice(t, cz, layer, want, a, a, KEV)
+    st, keep = ctx._stack(n, n, a, a, KEV, cz, layer, (0.0, 0.0), 2.0 / 3.0)
+    assert launched(ctx, lambda: msx.load().msx_multislice(ctx.h, C.byref(st), C.c_void_p(t.data_ptr()), None,
+                                                           C.c_void_p(psi.data_ptr()), 1, msx.F32, 1)) == 0
+    assert bool((psi == want.cpu()).all())
