@@ -116,8 +116,11 @@ MSX_API int msx_set_tuning(msx_ctx ctx, int nx, int ny, int prec, const msx_tuni
 MSX_API int msx_graph_stats(msx_ctx ctx, int64_t* captures, int64_t* replays);
 /* Without graphs, slice loops of few small waves (lengths 128 to 512) run as
  * one persistent kernel instead of two launches per slice: how many the
- * context has launched, and in how many calls one gave up waiting for its
- * work-groups (either may be NULL). */
+ * context has launched, and in how many calls one gave up (either may be
+ * NULL).  A loop gives up if its work-groups, which wait for each other, have
+ * not all been on the GPU for more than half a minute, as may happen where
+ * another process keeps it; the call then runs again from its incident waves
+ * without the loop, as do the context's later calls. */
 MSX_API int msx_loop_stats(msx_ctx ctx, int64_t* loops, int64_t* given_up);
 
 /* Kernel timing (the reference timed its loops with cudaEvents and printed

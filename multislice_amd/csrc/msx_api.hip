@@ -65,6 +65,7 @@ struct DevBuf {
         hipError_t e = hipMalloc(&p, bytes);
         if (e != hipSuccess) {
             p = nullptr;
+            (void)hipGetLastError();  // not for the launches of a caller that does without
             return fail(MSX_ENOMEM, "hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
         }
         n = bytes;
@@ -232,11 +233,14 @@ struct msx_ctx_s {
     size_t h_pin_cap = 0;
     // persistent slice loop: its flags and a layer list on the device, the
     // phase number the flags have reached, and the word a wait that gives up
-    // sets (pinned host memory, read after the stream is synchronised)
+    // sets (pinned host memory, read after the stream is synchronised).  A
+    // context in which one gave up uses the sweeps from then on
     DevBuf loopbuf, looplayers;
     unsigned loop_epoch = 0;
     int* loop_status = nullptr;
     int coop = -1;  // cooperative launches: not asked / no / yes
+    unsigned loop_polls = 1u << 26;  // polls before a wait gives up: over half a minute
+    bool loop_off = false;
     long long loops = 0, loops_given_up = 0;  // persistent loops launched, and calls in which one gave up
     int ensure_pinned(size_t n) {
         if (n <= h_pin_cap) return MSX_OK;
@@ -764,7 +768,6 @@ int slice_loop_body(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, 
 
 constexpr int kLoopFlags = 512;           // work-groups of a persistent loop at most
 constexpr int kLoopSlices = 6;
-constexpr unsigned kLoopSpin = 1u << 26;  // polls before a wait gives up: over half a minute
 
 // Where the persistent loop (msx_loop.hpp) replaces the sweeps: from 6 slices
 // on (2 slices 0.82-1.03x the sweeps' speed, 6 slices 0.96-1.11x) and up to 4M
@@ -780,14 +783,20 @@ constexpr unsigned kLoopSpin = 1u << 26;  // polls before a wait gives up: over 
 // 1527 / 1533.
 template <typename C> bool loop_wanted(msx_ctx ctx, int nx, int ny, int nb, int slices) {
     const msx_tuning* tu = ctx->tuning(nx, ny, sizeof(C) == 16 ? MSX_F64 : MSX_F32);
-    if (ctx->prof || !loop_built(nx, ny) || (tu && (tu->row_plan || tu->col_plan))) return false;
+    if (ctx->prof || ctx->loop_off || !loop_built(nx, ny) || (tu && (tu->row_plan || tu->col_plan))) return false;
     const long long px = (long long)nx * ny * nb;
     return slices >= kLoopSlices && px <= (sizeof(C) == 16 && nx == 512 ? 1LL << 20 : 1LL << 22);
 }
 
+// (the exchange past the caches is for memory of this device alone)
+template <typename C> bool loop_takes(msx_ctx ctx, const msx_stack* st, const C* psi, int nb, int slices) {
+    return !ctx->graphs && !is_oblique(st) && loop_wanted<C>(ctx, st->nx, st->ny, nb, slices) &&
+           msx_ctx_owns(ctx, psi, sizeof(C));
+}
+
 // Launches the loop `a` (its waves, slices and tables set) with a team of
 // work-groups per wave, as many as are resident; *done says whether it runs.
-// `passes`: barriers at most per wave.  The caller checks loop_failed() after
+// `passes`: barriers at most per wave.  The caller asks loop_gave_up() after
 // its stream synchronisation.
 template <typename C> int loop_go(msx_ctx ctx, int nx, int ny, LoopArgs<C>& a, unsigned passes, bool* done) {
     using Re = typename real_of<C>::type;
@@ -807,8 +816,8 @@ template <typename C> int loop_go(msx_ctx ctx, int nx, int ny, LoopArgs<C>& a, u
     // cleared once, and again before a word that was not used for long could
     // look newer than the phase it is compared with
     if (!ctx->loopbuf.p || ctx->loop_epoch > 1u << 30) {
-        CHK(ctx->loopbuf.ensure(sizeof(unsigned) * kLoopFlags));
-        HIPCHK(hipMemsetAsync(ctx->loopbuf.p, 0, sizeof(unsigned) * kLoopFlags, ctx->stream));
+        CHK(ctx->loopbuf.ensure(sizeof(unsigned) * (kLoopFlags + 1)));
+        HIPCHK(hipMemsetAsync(ctx->loopbuf.p, 0, sizeof(unsigned) * (kLoopFlags + 1), ctx->stream));
         ctx->loop_epoch = 0;
     }
     if (!ctx->loop_status) {
@@ -820,7 +829,8 @@ template <typename C> int loop_go(msx_ctx ctx, int nx, int ny, LoopArgs<C>& a, u
     a.inv = (Re)1 / ((Re)nx * (Re)ny);
     a.flags = static_cast<unsigned*>(ctx->loopbuf.p);
     a.epoch = ctx->loop_epoch;
-    a.spin = kLoopSpin;
+    a.dead = a.flags + kLoopFlags;
+    a.spin = ctx->loop_polls;
     a.status = ctx->loop_status;
     ctx->loop_epoch += passes * (unsigned)((a.nb + teams - 1) / teams);
     // a device or stream without room for a cooperative launch runs the sweeps
@@ -850,9 +860,7 @@ template <typename C>
 int persistent_loop(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, const C* trans, C* psi, int nb,
                     const C* src, long long src_bstride, int s0, int s1, int start, bool mixed_out, bool* done) {
     *done = false;
-    if (is_oblique(st) || !loop_wanted<C>(ctx, st->nx, st->ny, nb, s1 - s0)) return MSX_OK;
-    // the exchange past the caches is for memory of this device alone
-    if (!msx_ctx_owns(ctx, psi, sizeof(C))) return MSX_OK;
+    if (!loop_takes<C>(ctx, st, psi, nb, s1 - s0)) return MSX_OK;
     LoopArgs<C> a;
     std::memset(&a, 0, sizeof a);
     loop_tables(tb, &a);
@@ -883,13 +891,15 @@ int persistent_loop(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, 
     a.mixed = mixed_out;
     return loop_go<C>(ctx, st->nx, st->ny, a, 2u * (unsigned)(s1 - s0), done);
 }
-// after a synchronisation of the stream: a persistent loop whose barrier gave up
-int loop_failed(msx_ctx ctx) {
-    if (!ctx->loop_status || *ctx->loop_status == 0) return MSX_OK;
+// After a synchronisation of the stream: whether a persistent loop's barrier
+// gave up (something else held the GPU's work-group slots for half a minute).
+// The caller then starts again from its incident waves, by the sweeps.
+bool loop_gave_up(msx_ctx ctx) {
+    if (!ctx->loop_status || *ctx->loop_status == 0) return false;
     *ctx->loop_status = 0;
     ctx->loops_given_up++;
-    ctx->loopbuf.release();  // the next loop starts from cleared flags
-    return fail(MSX_EHIP, "slice loop: a barrier between its work-groups gave up");
+    ctx->loop_off = true;
+    return true;
 }
 
 // The slice loop, replayed from a cached hipGraph when graphs are enabled
@@ -899,10 +909,13 @@ int loop_failed(msx_ctx ctx) {
 // that fails falls back to launching the loop directly.
 template <typename C>
 int slice_loop(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, const C* trans, C* psi, int nb,
-               const C* src, long long src_bstride, int start, DetPlan* det, bool mixed_out = false) {
+               const C* src, long long src_bstride, int start, DetPlan* det, bool mixed_out = false,
+               bool loop = true) {
     if (!ctx->graphs && !det) {
         bool done = false;
-        CHK(persistent_loop<C>(ctx, st, tb, trans, psi, nb, src, src_bstride, 0, st->nslice, start, mixed_out, &done));
+        if (loop)
+            CHK(persistent_loop<C>(ctx, st, tb, trans, psi, nb, src, src_bstride, 0, st->nslice, start, mixed_out,
+                                   &done));
         if (done) return MSX_OK;
     } else if (!ctx->graphs) {
         // up to each checkpoint's slice, whose column sweep sums the detectors
@@ -1189,10 +1202,19 @@ int batch_class(msx_ctx ctx, const msx_job* jobs, std::vector<BatchItem>& g, std
     LoopJob<C>* hjb = reinterpret_cast<LoopJob<C>*>(hbase + o_jb);
     const C** hin = reinterpret_cast<const C**>(hbase + o_io);  // incident waves, then exit waves
     C** hout = reinterpret_cast<C**>(hbase + o_io) + nb;
+    loop = loop && !ctx->loop_off;
     for (int i = 0; i < nb; i++) {
         const msx_job& j = jobs[g[i].job];
         hin[i] = static_cast<const C*>(j.psi0 ? j.psi0 : j.psi);
         hout[i] = static_cast<C*>(j.psi);
+        if (loop && hin[i] == hout[i]) {
+            // the loop advances a wave in place: it reads a copy, in the wave's
+            // slot, which is kept until the loop has ended well
+            if (!(loop = ctx->wave.ensure(sizeof(C) * img * nb) == MSX_OK)) continue;
+            C* slot = static_cast<C*>(ctx->wave.p) + i * img;
+            HIPCHK(hipMemcpyAsync(slot, hout[i], sizeof(C) * img, hipMemcpyDeviceToDevice, ctx->stream));
+            hin[i] = slot;
+        }
         hjb[i] = LoopJob<C>{hout[i], hin[i], g[i].st->nslice, 0};
     }
     HIPCHK(hipMemcpyAsync(dbase, hbase, tot, hipMemcpyHostToDevice, ctx->stream));
@@ -1212,8 +1234,8 @@ int batch_class(msx_ctx ctx, const msx_job* jobs, std::vector<BatchItem>& g, std
         bool done = false;
         CHK(loop_go<C>(ctx, nx, ny, a, 2u * (unsigned)S, &done));
         if (done) {
-            if (sync) HIPCHK(hipStreamSynchronize(ctx->stream));
-            return MSX_OK;
+            HIPCHK(hipStreamSynchronize(ctx->stream));
+            if (!loop_gave_up(ctx)) return MSX_OK;
         }
     }
     // wave slots
@@ -1360,7 +1382,7 @@ template <typename C> int multislice_batch_impl(msx_ctx ctx, const msx_job* jobs
     const int nl = ctx->prof || loops ? 1 : std::min<int>(kLanes, (int)groups.size());
     if (nl <= 1) {
         for (auto& g : groups) CHK(batch_class<C>(ctx, jobs, g, keep, true, loops, direct));
-        return loop_failed(ctx);
+        return MSX_OK;
     }
     CHK(ctx->ensure_lanes(nl));
     // twiddle tables are shared: create them before any lane runs
@@ -1436,10 +1458,34 @@ int multislice_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const v
     }
     SliceTables<C> tb;
     CHK(build_tables<C>(ctx, st, true, &tb));
-    CHK(slice_loop<C>(ctx, st, tb, t_dev, w_dev, nwave, s_dev, 0, 0, nullptr));
-    if (where == MSX_HOST) HIPCHK(hipMemcpyAsync(psi, w_dev, wbytes, hipMemcpyDeviceToHost, ctx->stream));
+    // The loop advances the waves in place; where that would overwrite the only
+    // incident ones it reads a copy, kept until the loop has ended well.
+    long long stride = 0;
+    bool loop = true;
+    if (where == MSX_DEVICE && loop_takes<C>(ctx, st, w_dev, nwave, st->nslice)) {
+        const bool apart = s_dev && (s_dev + img <= w_dev || w_dev + img * nwave <= s_dev);
+        const C* in = s_dev ? s_dev : w_dev;
+        const size_t bytes = s_dev ? sizeof(C) * img : wbytes;
+        loop = apart || ctx->wave.ensure(bytes) == MSX_OK;
+        if (!apart && loop) {
+            HIPCHK(hipMemcpyAsync(ctx->wave.p, in, bytes, hipMemcpyDeviceToDevice, ctx->stream));
+            stride = s_dev ? 0 : img;
+            s_dev = static_cast<const C*>(ctx->wave.p);
+        }
+    }
+    CHK(slice_loop<C>(ctx, st, tb, t_dev, w_dev, nwave, s_dev, stride, 0, nullptr, false, loop));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    return loop_failed(ctx);
+    if (loop_gave_up(ctx)) {
+        if (where == MSX_HOST && !psi0)
+            HIPCHK(hipMemcpyAsync(w_dev, psi, wbytes, hipMemcpyHostToDevice, ctx->stream));
+        CHK(slice_loop<C>(ctx, st, tb, t_dev, w_dev, nwave, s_dev, stride, 0, nullptr));
+        HIPCHK(hipStreamSynchronize(ctx->stream));
+    }
+    if (where == MSX_HOST) {
+        HIPCHK(hipMemcpyAsync(psi, w_dev, wbytes, hipMemcpyDeviceToHost, ctx->stream));
+        HIPCHK(hipStreamSynchronize(ctx->stream));
+    }
+    return MSX_OK;
 }
 
 // msx_multislice with the records of a thickness series.  One device block
@@ -1669,7 +1715,8 @@ int stem_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_pro
     std::vector<double> res((size_t)nck * ndet * nprobe);
     HIPCHK(hipMemcpyAsync(res.data(), o_dev, obytes, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    CHK(loop_failed(ctx));
+    if (loop_gave_up(ctx))
+        return stem_impl<C>(ctx, st, trans, pr, pos, nprobe, det, ndet, ck, nck, weight, accumulate, out, batch, where);
     for (size_t i = 0; i < res.size(); i++) out[i] = (accumulate ? out[i] : 0.0) + weight * res[i];
     return MSX_OK;
 }
@@ -1904,7 +1951,9 @@ int partial_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_
     }
     if (where == MSX_HOST) HIPCHK(hipMemcpyAsync(image, pix, ibytes, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    return loop_failed(ctx);
+    if (loop_gave_up(ctx))
+        return partial_impl<C>(ctx, st, trans, lens, acmin, acmax, sigmaf, dfdelt, batch, image, nangles, nsteps, where);
+    return MSX_OK;
 }
 
 // host binning of atoms for the splat kernel
@@ -2550,6 +2599,12 @@ MSX_API int msx_loop_stats(msx_ctx ctx, int64_t* loops, int64_t* given_up) {
     if (!ctx) return fail(MSX_ESTATE, "ctx is NULL");
     if (loops) *loops = ctx->loops;
     if (given_up) *given_up = ctx->loops_given_up;
+    return MSX_OK;
+}
+
+int msx_test_loop_polls(msx_ctx ctx, unsigned polls) {
+    if (!ctx) return fail(MSX_ESTATE, "ctx is NULL");
+    ctx->loop_polls = polls;
     return MSX_OK;
 }
 

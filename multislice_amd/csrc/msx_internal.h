@@ -318,6 +318,8 @@ int fail(int code, const char* fmt, ...);
 struct msx_ctx_s;
 int msx_ctx_device(const msx_ctx_s* ctx);
 hipStream_t msx_ctx_stream(const msx_ctx_s* ctx);
+// for tests: polls before a wait of the persistent slice loop gives up
+extern "C" __attribute__((visibility("default"))) int msx_test_loop_polls(msx_ctx_s* ctx, unsigned polls);
 // whether q is memory of the context's own device, aligned as given: what its
 // kernels may read and write in place
 bool msx_ctx_owns(const msx_ctx_s* ctx, const void* q, size_t align);

@@ -20,7 +20,9 @@
 //
 // Every wait ends: the launch is cooperative (all work-groups resident, or
 // the launch fails), and a work-group that polls longer than `spin` times
-// raises `status` and leaves, after which the others run out as well.
+// raises `status` and `dead` and leaves, after which the others run out as
+// well; loops launched before the host has seen it leave at their first
+// barrier.  The host then runs the call again by the sweeps.
 #pragma once
 #include "msx_sweep.hpp"
 
@@ -66,7 +68,8 @@ template <typename C> struct LoopArgs {
     unsigned* flags;        // [teams][team] phase numbers, all at most `epoch`
     unsigned epoch;
     unsigned spin;          // polls before a wait gives up
-    int* status;            // set to 1 by a wait that gave up
+    unsigned* dead;         // set by a wait that gave up, on the device ..
+    int* status;            // .. and for the host
 };
 
 template <typename C, int NX, int NY> struct LoopShape {
@@ -99,7 +102,7 @@ __global__ __launch_bounds__((LoopShape<C, NX, NY>::BT)) void slice_loop_kernel(
     const int tid = threadIdx.x;
     const int team = (int)blockIdx.x / p.team, m = (int)blockIdx.x % p.team, nteam = (int)gridDim.x / p.team;
     unsigned* const flags = p.flags + (size_t)team * p.team;
-    if (tid == 0) gave_up = 0;
+    const unsigned dead = __hip_atomic_load(p.dead, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
     // row phase: line lw, position t
     const int lw = tid / T, t = tid % T;
@@ -149,12 +152,16 @@ __global__ __launch_bounds__((LoopShape<C, NX, NY>::BT)) void slice_loop_kernel(
         asm volatile("" ::: "memory");
         lds_barrier();
         if (gave_up) {
-            if (tid == 0) *p.status = 1;
+            if (tid == 0) {
+                __hip_atomic_store(p.dead, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                *p.status = 1;
+            }
             return false;
         }
         return true;
     };
 
+    if (tid == 0) gave_up = dead != 0;  // (read after the first barrier)
     for (int b = team; b < p.nb; b += nteam) {
         C* img = p.psi + (long long)b * NX * NY;
         const C* in0 = p.src ? p.src + b * p.src_bstride : img;
