@@ -231,11 +231,11 @@ struct msx_ctx_s {
     std::vector<int> h_cnt, h_fill;
     AtomRec* h_pin = nullptr;
     size_t h_pin_cap = 0;
-    // persistent slice loop: its flags and a layer list on the device, the
-    // phase number the flags have reached, and the word a wait that gives up
-    // sets (pinned host memory, read after the stream is synchronised).  A
-    // context in which one gave up uses the sweeps from then on
-    DevBuf loopbuf, looplayers;
+    // persistent slice loop: its flags on the device, the phase number the
+    // flags have reached, and the word a wait that gives up sets (pinned host
+    // memory, read after the stream is synchronised).  A context in which one
+    // gave up uses the sweeps from then on
+    DevBuf loopbuf;
     unsigned loop_epoch = 0;
     int* loop_status = nullptr;
     int coop = -1;  // cooperative launches: not asked / no / yes
@@ -321,7 +321,7 @@ struct msx_ctx_s {
         for (auto& kv : tw64) kv.second.release();
         drop_graphs();
         for (DevBuf* b : {&wave, &wave2, &trans, &aux, &tabs, &partial, &outbuf, &atoms, &cells, &vtmp, &curvebuf, &radtab,
-                           &radcoef, &binbuf, &series, &unitbuf, &loopbuf, &looplayers})
+                           &radcoef, &binbuf, &series, &unitbuf, &loopbuf})
             b->release();
         for (Lane& l : lanes) {
             l.wave.release();
@@ -363,6 +363,9 @@ template <typename C> struct SliceTables {
     const C* px = nullptr;
     const C* py = nullptr;
     std::vector<int> which;
+    // (layer, factors) of every slice for the persistent loop, or null: slice s
+    // is layer s and all layers take the same factors
+    const int2* slices = nullptr;
     float k2max = 0.f;
     Band band;  // the y columns with ky2 < k2max
     // twiddles of the x and y transforms; null: the context's cached tables
@@ -377,9 +380,10 @@ template <typename C> struct HostTables {
     std::vector<float> kx2, ky2;
     std::vector<C> px, py;
     std::vector<int> which;
+    std::vector<int2> slices;  // SliceTables::slices, empty for null
     // per_layer: the block's size with factors for every layer (the bound of
-    // callers with a fixed block, whatever the thicknesses)
-    size_t o_ky = 0, o_px = 0, o_py = 0, tot = 0, per_layer = 0;
+    // callers with a fixed block, whatever the thicknesses; they take no list)
+    size_t o_ky = 0, o_px = 0, o_py = 0, o_sl = 0, tot = 0, per_layer = 0;
 };
 
 inline size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -400,7 +404,7 @@ template <typename C> void prop_factors(int n, double a, double cz, double lam, 
 // One pair of factor arrays per distinct slice thickness: most stacks have a
 // single one, and evaluating 2 x 256 sines and cosines per layer took 0.54 of
 // the 1.47 ms of an 80-layer 256^2 call.
-template <typename C> void host_tables(const msx_stack* st, bool with_prop, HostTables<C>* h) {
+template <typename C> void host_tables(const msx_stack* st, bool with_prop, HostTables<C>* h, bool list = false) {
     const int nx = st->nx, ny = st->ny, nl = with_prop ? st->nlayer : 0;
     h->kx2 = k2_table(nx, st->ax);
     h->ky2 = k2_table(ny, st->by);
@@ -430,6 +434,16 @@ template <typename C> void host_tables(const msx_stack* st, bool with_prop, Host
     h->o_px = h->o_ky + al256(sizeof(float) * ny);
     h->o_py = h->o_px + al256(sizeof(C) * h->px.size());
     h->tot = h->o_py + al256(sizeof(C) * h->py.size() + 1);
+    if (list && nl > 0) {
+        bool straight = true;
+        for (int s = 0; s < st->nslice && straight; s++) straight = st->layer[s] == s && h->which[s] == 0;
+        if (!straight) {
+            h->slices.resize(st->nslice);
+            for (int s = 0; s < st->nslice; s++) h->slices[s] = make_int2(st->layer[s], h->which[st->layer[s]]);
+        }
+        h->o_sl = h->tot;
+        h->tot += sizeof(int2) * h->slices.size();
+    }
     h->per_layer = h->o_px + al256(sizeof(C) * (size_t)nl * nx) + al256(sizeof(C) * (size_t)nl * ny + 1);
 }
 
@@ -443,6 +457,7 @@ int upload_tables(msx_ctx ctx, const msx_stack* st, const HostTables<C>& h, char
     std::memcpy(block.data() + h.o_ky, h.ky2.data(), sizeof(float) * ny);
     std::memcpy(block.data() + h.o_px, h.px.data(), sizeof(C) * h.px.size());
     std::memcpy(block.data() + h.o_py, h.py.data(), sizeof(C) * h.py.size());
+    if (!h.slices.empty()) std::memcpy(block.data() + h.o_sl, h.slices.data(), sizeof(int2) * h.slices.size());
     HIPCHK(hipMemcpyAsync(base, block.data(), h.tot, hipMemcpyHostToDevice, ctx->stream));
     // the host block must outlive the async copy
     HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -451,6 +466,7 @@ int upload_tables(msx_ctx ctx, const msx_stack* st, const HostTables<C>& h, char
     out->px = reinterpret_cast<const C*>(base + h.o_px);
     out->py = reinterpret_cast<const C*>(base + h.o_py);
     out->which = h.which;
+    out->slices = h.slices.empty() ? nullptr : reinterpret_cast<const int2*>(base + h.o_sl);
     out->k2max = k2max_of(nx, ny, st->ax, st->by, st->bw);
     out->band = band_limits(h.ky2.data(), ny, out->k2max);
     ctx->band = band_fraction(h.ky2.data(), ny, out->k2max);
@@ -460,7 +476,7 @@ int upload_tables(msx_ctx ctx, const msx_stack* st, const HostTables<C>& h, char
 template <typename C>
 int build_tables(msx_ctx ctx, const msx_stack* st, bool with_prop, SliceTables<C>* out) {
     HostTables<C> h;
-    host_tables<C>(st, with_prop, &h);
+    host_tables<C>(st, with_prop, &h, true);
     CHK(ctx->tabs.ensure(h.tot));
     return upload_tables<C>(ctx, st, h, static_cast<char*>(ctx->tabs.p), out);
 }
@@ -870,19 +886,7 @@ int persistent_loop(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, 
     a.trans = trans;
     a.px = tb.px;
     a.py = tb.py;
-    // (layer, factors) of every slice, unless slice s is layer s and all
-    // layers take the same factors
-    bool straight = true;
-    for (int s = s0; s < s1 && straight; s++) straight = st->layer[s] == s && tb.which[s] == 0;
-    if (!straight) {
-        std::vector<int2> sl(st->nslice);
-        for (int s = 0; s < st->nslice; s++) sl[s] = make_int2(st->layer[s], tb.which[st->layer[s]]);
-        CHK(ctx->looplayers.ensure(sizeof(int2) * sl.size()));
-        HIPCHK(hipMemcpyAsync(ctx->looplayers.p, sl.data(), sizeof(int2) * sl.size(), hipMemcpyHostToDevice,
-                              ctx->stream));
-        HIPCHK(hipStreamSynchronize(ctx->stream));  // sl must outlive the copy
-        a.slices = static_cast<const int2*>(ctx->looplayers.p);
-    }
+    a.slices = tb.slices;
     a.s0 = s0;
     a.s1 = s1;
     a.nb = nb;
