@@ -783,25 +783,31 @@ int slice_loop_body(msx_ctx ctx, const msx_stack* st, const SliceTables<C>& tb, 
 }
 
 constexpr int kLoopFlags = 512;           // work-groups of a persistent loop at most
-constexpr int kLoopSlices = 6;
 
-// Where the persistent loop (msx_loop.hpp) replaces the sweeps: from 6 slices
-// on (2 slices 0.82-1.03x the sweeps' speed, 6 slices 0.96-1.11x) and up to 4M
-// pixels of waves.  Whole calls of 40 slices, us, sweeps / loop, FP32: 128^2 1
-// wave 583 / 483, 64 waves 831 / 542, 256 waves 1580 / 1102; 256^2 1 wave 616 /
-// 524, 13 waves 801 / 616, 64 waves 1597 / 1272; 384^2 1 wave 899 / 704, 24 waves
-// 2031 / 1866, 32 waves 1247 / 1331 (20 slices); 512^2 1 wave 730 / 679, 8 waves
-// 843 / 664 (20 slices), 16 waves 1034 / 886, 32 waves 1427 / 1383, 64 waves
-// 2020 / 2345: past that the waves keep the sweeps' launches full, and the
-// write-through exchange costs more than the launches.  FP64 gains the same
-// (256^2 13 waves 1092 / 853, 384^2 24 waves 3282 / 2620) but for 512-element
-// columns, whose tiles are 4 wide: 1-2 waves 838 / 756 and 958 / 831, 6 waves
-// 1527 / 1533.
+// Where the persistent loop (msx_loop.hpp) replaces the sweeps: up to 4M pixels
+// of waves, past which they keep the sweeps' launches full and the write-through
+// exchange costs more than the launches (512^2, 20 slices: 16 waves 1034 / 886
+// us sweeps / loop, 32 waves 1427 / 1383, 64 waves 2020 / 2345; in FP64 columns of
+// 512, in tiles of 4, up to 1M: 6 waves 1527 / 1533).
+//  A loop costs about 40 us more than two launches before its first slice and
+// gains per slice.  From 8 MiB of waves on it has won at 6 slices (1.00 to 1.47
+// times the sweeps' speed; in FP64 512^2 of 3 waves 0.96, 512 x 256 of 6 0.98),
+// with fewer waves at 16 (256^2 1 wave: 6 slices 0.97, 12 1.00, 16 1.02, 80 1.12; 384 x 128: 1.08, 1.17,
+// 1.23, 1.34; 384 x 512: 0.94, 1.03, 1.01, 1.07).  Where the sweeps are short for
+// the barriers of the team it does not win at all until the waves are larger:
+// FP32 columns of 512 (1 wave of 80 slices: 512 x 128 0.87, x 256 1.00, x 384
+// 0.92, 512^2 1.01; of 4 MiB: 1.00, 1.13, 1.03, 1.08), 128 x 256 (1 to 8 waves
+// 0.94-1.05, 16 waves 1.05; FP64 0.94-1.05, 1.22), FP64 512 x 128 (1.00; of 4 MiB
+// 1.09).
 template <typename C> bool loop_wanted(msx_ctx ctx, int nx, int ny, int nb, int slices) {
-    const msx_tuning* tu = ctx->tuning(nx, ny, sizeof(C) == 16 ? MSX_F64 : MSX_F32);
+    constexpr bool f32 = sizeof(C) == 8;
+    const msx_tuning* tu = ctx->tuning(nx, ny, f32 ? MSX_F32 : MSX_F64);
     if (ctx->prof || ctx->loop_off || !loop_built(nx, ny) || (tu && (tu->row_plan || tu->col_plan))) return false;
-    const long long px = (long long)nx * ny * nb;
-    return slices >= kLoopSlices && px <= (sizeof(C) == 16 && nx == 512 ? 1LL << 20 : 1LL << 22);
+    const long long px = (long long)nx * ny * nb, mib = px * (long long)sizeof(C) >> 20;
+    if (px > (!f32 && nx == 512 ? 1LL << 20 : 1LL << 22)) return false;
+    const bool narrow = nx == 512 && ny == 128;
+    if (((f32 && nx == 512) || narrow || (nx == 128 && ny == 256)) && mib < (f32 && narrow ? 8 : 4)) return false;
+    return slices >= (mib >= 8 ? 6 : 16);
 }
 
 // (the exchange past the caches is for memory of this device alone)

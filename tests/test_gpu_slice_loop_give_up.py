@@ -77,7 +77,7 @@ def test_exit_waves(ctx, short, form, f64):
 def test_stem(ctx, short):
     t = trans()
     pos = np.random.default_rng(0).uniform(0, A, (9, 2))
-    args = (t, CZ, LAYER, A, A, KEV, dict(alpha_max=0.02), pos, [(0, 0.4), (1.0, 3.0)], [9, NS])
+    args = (t, CZ, LAYER, A, A, KEV, dict(alpha_max=0.02), pos, [(0, 0.4), (1.0, 3.0)], [18, NS])
     ctx.set_graphs(True)
     want = ctx.stem(*args, batch=4)
     ctx.set_graphs(False)

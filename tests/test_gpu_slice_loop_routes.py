@@ -27,7 +27,7 @@ def launched(ctx, fn):
 
 
 @pytest.mark.parametrize("f64", [False, True])
-@pytest.mark.parametrize("n,nwave", [(128, 1), (128, 256), (256, 5), (384, 2), (512, 1)])
+@pytest.mark.parametrize("n,nwave", [(128, 1), (128, 256), (256, 5), (384, 2), (512, 2)])
 def test_exit_waves(ctx, n, nwave, f64):
     import torch
     ns, a = 20, 0.1 * n
@@ -46,6 +46,46 @@ def test_exit_waves(ctx, n, nwave, f64):
     ctx.profile(False)
 
 
+@pytest.mark.parametrize("f64", [False, True])
+@pytest.mark.parametrize("nx", [128, 256, 384, 512])
+@pytest.mark.parametrize("ny", [128, 256, 384, 512])
+def test_every_shape_equals_sweeps(ctx, nx, ny, f64):
+    """One kernel per shape and precision, with as many waves as the rule asks
+    for and one more: bits of the sweeps (graphs), repeated layers of unequal
+    thickness, and with 16 slices and no loop with 15, or 6 and 5 from 8 MiB on."""
+    import torch
+    size = nx * ny * (16 if f64 else 8)
+    few = 1
+    if (nx == 512 and not f64) or (nx, ny) in ((128, 256), (512, 128)):
+        few = (8 if (nx, ny, f64) == (512, 128, False) else 4) * 2**20 // size
+        few += few * size < 4 * 2**20  # (not a whole number of waves)
+    many = -(-8 * 2**20 // size)
+    a, b = 0.1 * nx, 0.1 * ny
+    g = torch.Generator(device="cuda").manual_seed(nx + 7 * ny)
+    ph = torch.rand((3, nx, ny), generator=g, device="cuda", dtype=torch.float64 if f64 else torch.float32)
+    t = torch.polar(torch.ones_like(ph), ph)
+    first = torch.randn((max(few, many) + 1, nx, ny), dtype=t.dtype, device="cuda", generator=g)
+
+    def run(n, ns):
+        w = first[:n].clone()
+        ctx.multislice(t, [2.0, 1.5, 2.0], np.arange(ns) % 3, w, a, b, KEV)
+        return w
+    for n, ns in ((few, 16), (few + 1, 17), (many, 6), (many + 1, 7)):
+        if n < many and n * size >= 8 * 2**20:
+            continue
+        ctx.set_graphs(True)
+        want = run(n, ns)
+        ctx.set_graphs(False)
+        got = []
+        assert launched(ctx, lambda: got.append(run(n, ns))) == 1
+        assert bool((got[0] == want).all())
+    assert launched(ctx, lambda: run(many, 5)) == 0
+    if few < many:
+        assert launched(ctx, lambda: run(few, 15)) == 0
+    if few > 1:
+        assert launched(ctx, lambda: run(few - 1, 40)) == 0
+
+
 def test_lengths_without_a_loop(ctx):
     import torch
     for n in (64, 768):
@@ -56,11 +96,11 @@ def test_lengths_without_a_loop(ctx):
 
 def test_stem_partial_coherence_and_job_sets(ctx):
     import torch
-    n, ns, a = 128, 20, 12.8
+    n, ns, a = 128, 40, 12.8
     t, cz, layer = trans(n, ns), np.full(ns, 2.0), np.arange(ns)
     pos = np.random.default_rng(0).uniform(0, a, (9, 2))
     # a loop up to each checkpoint's slice, for each of three batches
-    assert launched(ctx, lambda: ctx.stem(t, cz, layer, a, a, KEV, dict(alpha_max=0.02), pos, [(0, 1.0)], [10, 20],
+    assert launched(ctx, lambda: ctx.stem(t, cz, layer, a, a, KEV, dict(alpha_max=0.02), pos, [(0, 1.0)], [20, 40],
                                           batch=3)) == 6
     lens = dict(cs=1e7, df=500.0, aobj=0.02)
     assert launched(ctx, lambda: ctx.partial_coherence(t, cz, layer, a, a, KEV, lens, 0.0, 5e-3, 30.0, 15.0)) == 1
