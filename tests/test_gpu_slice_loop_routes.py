@@ -94,19 +94,35 @@ def test_lengths_without_a_loop(ctx):
         assert launched(ctx, lambda: ctx.multislice(t, np.full(20, 2.0), np.arange(20), psi, 10.0, 10.0, KEV)) == 0
 
 
+def taken(ctx, fn, loops):
+    """fn() by loops, so many of them, and by the sweeps (profiled): the same bits."""
+    got = []
+    assert launched(ctx, lambda: got.append(fn())) == loops
+    ctx.profile(True)
+    assert launched(ctx, lambda: got.append(fn())) == 0
+    ctx.profile(False)
+    assert all(bool((x == y).all()) for x, y in zip(*got))
+
+
 def test_stem_partial_coherence_and_job_sets(ctx):
     import torch
     n, ns, a = 128, 40, 12.8
     t, cz, layer = trans(n, ns), np.full(ns, 2.0), np.arange(ns)
-    pos = np.random.default_rng(0).uniform(0, a, (9, 2))
+    pos = np.random.default_rng(0).uniform(0, a, (8, 2))
     # a loop up to each checkpoint's slice, for each of three batches
-    assert launched(ctx, lambda: ctx.stem(t, cz, layer, a, a, KEV, dict(alpha_max=0.02), pos, [(0, 1.0)], [20, 40],
-                                          batch=3)) == 6
+    taken(ctx, lambda: ctx.stem(t, cz, layer, a, a, KEV, dict(alpha_max=0.02), pos, [(0, 1.0), (1.0, 3.0)], [20, 40],
+                                batch=3), 6)
     lens = dict(cs=1e7, df=500.0, aobj=0.02)
-    assert launched(ctx, lambda: ctx.partial_coherence(t, cz, layer, a, a, KEV, lens, 0.0, 5e-3, 30.0, 15.0)) == 1
-    jobs = [dict(trans=t, psi=torch.ones((n, n), dtype=t.dtype, device="cuda"), ax=a, by=a, kev=KEV, cz=cz,
-                 layer=layer) for _ in range(3)]
-    assert launched(ctx, lambda: ctx.multislice_batch(jobs)) == 1
+    taken(ctx, lambda: ctx.partial_coherence(t, cz, layer, a, a, KEV, lens, 0.0, 5e-3, 30.0, 15.0)[:1], 1)
+
+    def job_set():  # one class with uneven ends, more waves than one team; another cell
+        g = torch.Generator(device="cuda").manual_seed(1)
+        jobs = [dict(trans=t, psi=torch.randn((n, n), dtype=t.dtype, device="cuda", generator=g), ax=a,
+                     by=a + (k == 5), kev=KEV + k % 2, cz=cz, layer=layer[:ns - k]) for k in range(24)]
+        jobs[3]["psi0"] = torch.ones_like(jobs[3]["psi"])
+        ctx.multislice_batch(jobs)
+        return [j["psi"] for j in jobs]
+    taken(ctx, job_set, 2)
 
 
 def test_waves_in_pinned_memory(ctx):
