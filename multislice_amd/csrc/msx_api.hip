@@ -25,6 +25,7 @@ using namespace msx;
 namespace msx {
 
 thread_local std::string g_err;
+thread_local size_t t_alloc_limit = 0;
 
 int fail(int code, const char* fmt, ...) {
     char buf[1024];
@@ -62,10 +63,9 @@ struct DevBuf {
         if (p) hipFree(p);
         p = nullptr;
         n = 0;
-        hipError_t e = hipMalloc(&p, bytes);
+        hipError_t e = device_alloc(&p, bytes);
         if (e != hipSuccess) {
             p = nullptr;
-            (void)hipGetLastError();  // not for the launches of a caller that does without
             return fail(MSX_ENOMEM, "hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
         }
         n = bytes;
@@ -1641,7 +1641,8 @@ int stem_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_pro
     const long long img = (long long)nx * ny;
     const msx_tuning* tu = ctx->tuning(nx, ny, sizeof(Re) == 8 ? MSX_F64 : MSX_F32);
     if (batch <= 0 && tu && tu->batch > 0) batch = tu->batch;
-    if (batch <= 0) batch = default_batch<C>(nx, ny, nprobe);
+    const bool chosen = batch > 0;
+    if (!chosen) batch = default_batch<C>(nx, ny, nprobe);
     batch = std::min(batch, nprobe);
     const C* t_dev = static_cast<const C*>(trans);
     if (where == MSX_HOST) {
@@ -1650,6 +1651,8 @@ int stem_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_pro
         HIPCHK(hipMemcpyAsync(ctx->trans.p, trans, tbytes, hipMemcpyHostToDevice, ctx->stream));
         t_dev = static_cast<const C*>(ctx->trans.p);
     }
+    // (the smaller batch of other grids where there is no room for this one)
+    if (!chosen && batch > 256 && ctx->wave.ensure(sizeof(C) * img * batch) != MSX_OK) batch = 256;
     CHK(ctx->wave.ensure(sizeof(C) * img * batch));
     C* w_dev = static_cast<C*>(ctx->wave.p);
     const int groups = col_groups<C>(nx, ny, tu ? tu->col_tile : 0);
@@ -1861,7 +1864,7 @@ int partial_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_
     // most of the GPU idle: 13 waves of 256^2 at 21 steps with 80 slices before
     // them: 1820 us per call with a launch pair per step, 1536 with one for all)
     const int nd = (int)off.size();
-    const int per = (int)std::max(1LL, std::min<long long>(nd, (320LL << 20) / (long long)(sizeof(C) * img) / batch));
+    int per = (int)std::max(1LL, std::min<long long>(nd, (320LL << 20) / (long long)(sizeof(C) * img) / batch));
     const C* t_dev = static_cast<const C*>(trans);
     if (where == MSX_HOST) {
         const size_t tbytes = sizeof(C) * img * st->nlayer;
@@ -1870,10 +1873,8 @@ int partial_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_
         t_dev = static_cast<const C*>(ctx->trans.p);
     }
     CHK(ctx->wave.ensure(sizeof(C) * img * batch));
-    CHK(ctx->wave2.ensure(sizeof(C) * img * batch * per));
     CHK(ctx->vtmp.ensure(sizeof(Re) * img * batch));
     C* w = static_cast<C*>(ctx->wave.p);
-    C* w2 = static_cast<C*>(ctx->wave2.p);
     Re* ib = static_cast<Re*>(ctx->vtmp.p);
     // image | illumination angles | defocus of every step | weight of every step
     const size_t ibytes = sizeof(double) * img, iq_off = al256(ibytes), df_off = iq_off + al256(sizeof(int2) * iq.size()),
@@ -1898,6 +1899,10 @@ int partial_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_
     const C *twx, *twy;
     CHK(ctx->twiddles<C>(nx, &twx));
     CHK(ctx->twiddles<C>(ny, &twy));
+    // (one step at a time where there is no room for more)
+    if (per > 1 && ctx->wave2.ensure(sizeof(C) * img * batch * per) != MSX_OK) per = 1;
+    CHK(ctx->wave2.ensure(sizeof(C) * img * batch * per));
+    C* w2 = static_cast<C*>(ctx->wave2.p);
     const double lam = msx_wavelength(st->kev);
     const float kap_hi = (float)((lens->aobj / lam) * (lens->aobj / lam));
     // columns with ky2 > kap_hi are zero after the lens and those with
@@ -2454,6 +2459,13 @@ bool msx_ctx_owns(const msx_ctx_s* ctx, const void* q, size_t align) {
     }
     return at.type == hipMemoryTypeDevice && at.device == ctx->device && (uintptr_t)q % align == 0;
 }
+hipError_t device_alloc(void** p, size_t bytes) {
+    if (t_alloc_limit && bytes > t_alloc_limit) return hipErrorOutOfMemory;
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+void msx_test_alloc_limit(size_t bytes) { t_alloc_limit = bytes; }
 int msx_ctx_scratch(msx_ctx_s* ctx, size_t bytes, void** out) {
     CHK(ctx->unitbuf.ensure(bytes));
     *out = ctx->unitbuf.p;

@@ -318,6 +318,10 @@ int fail(int code, const char* fmt, ...);
 struct msx_ctx_s;
 int msx_ctx_device(const msx_ctx_s* ctx);
 hipStream_t msx_ctx_stream(const msx_ctx_s* ctx);
+// hipMalloc; a failure leaves no error behind for later launches to report
+hipError_t device_alloc(void** p, size_t bytes);
+// for tests: allocations of the calling thread larger than `bytes` fail (0: none)
+extern "C" __attribute__((visibility("default"))) void msx_test_alloc_limit(size_t bytes);
 // for tests: polls before a wait of the persistent slice loop gives up
 extern "C" __attribute__((visibility("default"))) int msx_test_loop_polls(msx_ctx_s* ctx, unsigned polls);
 // whether q is memory of the context's own device, aligned as given: what its

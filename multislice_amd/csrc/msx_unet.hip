@@ -67,7 +67,7 @@ struct msx_unet_s {
     float* ws = nullptr;
     size_t ws_bytes = 0;
     double* partial = nullptr;
-    __bf16* pk = nullptr;   // packed 3x3 weights: every layer's kFwd, then every layer's kBwdData
+    __bf16* pk = nullptr;   // packed 3x3 weights: every layer's kFwd, then every layer's kBwdData (null: no room)
     std::vector<size_t> pk_off[2];
     size_t pk_n[2] = {0, 0};
     bool pk_ok[2] = {false, false};  // packed since the weights last changed
@@ -191,7 +191,7 @@ struct msx_unet_s {
     const __bf16* packed(int mode, int i) const { return pk + (mode == kFwd ? 0 : pk_n[kFwd]) + pk_off[mode][i]; }
     // pack every 3x3 layer for `mode` if the weights have changed since
     int pack(int mode) {
-        if (pk_ok[mode]) return MSX_OK;
+        if (!pk || pk_ok[mode]) return MSX_OK;
         PackArgs a{};
         a.w = params();
         a.out = pk + (mode == kFwd ? 0 : pk_n[kFwd]);
@@ -222,7 +222,7 @@ struct msx_unet_s {
         return a;
     }
     // does layer i at level l run the packed kernel?
-    bool packs(int i, int l) { return convs[i].ks == 3 && conv3_fits(conv_args(i, wn, l)); }
+    bool packs(int i, int l) { return pk && convs[i].ks == 3 && conv3_fits(conv_args(i, wn, l)); }
     // a: the extra outputs (pool, skip, up) of the packed kernel or the
     // residual of the head
     int conv_fwd(int i, int l, const float* x, float* y, const ConvArgs* extra = nullptr) {
@@ -272,25 +272,33 @@ struct msx_unet_s {
     // nothing that follows and no layer waits for them, while a layer by itself
     // leaves most of the chip idle: two launches for all layers of a
     // step take 101 us instead of 312 for two per layer (16 32^2 images).
+    // Without room for the slices of all, one layer after the other.
     int weight_grads() {
-        if (wg_need > wscr_n) {
-            UHIP(hipStreamSynchronize(stream()));
-            if (wscr) hipFree(wscr);
-            wscr = nullptr;
-            wscr_n = 0;
-            UHIP(hipMalloc(&wscr, wg_need * sizeof(float)));
-            wscr_n = wg_need;
-        }
-        float* part = wscr;
-        for (int i = 0; i < nwg; i++) {
-            wg[i].a.partial = part;
-            part += conv_wgrad_scratch(wg[i].ks, wg[i].a);
-        }
         const int n = nwg;
         nwg = 0;
+        size_t most = 0;
+        for (int i = 0; i < n; i++) most = std::max(most, conv_wgrad_scratch(wg[i].ks, wg[i].a));
+        const bool all = wgrad_room(wg_need);
         wg_need = 0;
-        UHIP(launch_wgrad(wg, n, stream()));
+        if (!all && !wgrad_room(most)) return fail(MSX_ENOMEM, "weight gradients: %zu floats of scratch", most);
+        float* part = wscr;
+        for (int i = 0; i < n; i++) {
+            wg[i].a.partial = part;
+            if (all) part += conv_wgrad_scratch(wg[i].ks, wg[i].a);
+            else UHIP(launch_wgrad(&wg[i], 1, stream()));
+        }
+        if (all) UHIP(launch_wgrad(wg, n, stream()));
         return MSX_OK;
+    }
+    bool wgrad_room(size_t floats) {
+        if (floats <= wscr_n) return true;
+        (void)hipStreamSynchronize(stream());
+        if (wscr) hipFree(wscr);
+        wscr = nullptr;
+        wscr_n = 0;
+        if (device_alloc(reinterpret_cast<void**>(&wscr), floats * sizeof(float)) != hipSuccess) return false;
+        wscr_n = floats;
+        return true;
     }
 
     // forward from x; leaves the head's output in z, or with y set writes
@@ -476,7 +484,11 @@ MSX_API int msx_unet_create_in(msx_ctx ctx, int levels, int base_channels, int i
     }
     net->plan_packs();
     hipError_t e = hipMalloc(&net->pbuf, 4 * off * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&net->pk, (net->pk_n[kFwd] + net->pk_n[kBwdData]) * sizeof(__bf16));
+    // (a network without room for the packed weights runs the general kernels)
+    if (e == hipSuccess &&
+        device_alloc(reinterpret_cast<void**>(&net->pk), (net->pk_n[kFwd] + net->pk_n[kBwdData]) * sizeof(__bf16)) !=
+            hipSuccess)
+        net->pk = nullptr;
     if (e == hipSuccess) e = hipMalloc(&net->partial, kSqBlocks * sizeof(double));
     if (e == hipSuccess) e = hipMemcpy(net->pbuf, p.data(), off * sizeof(float), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(net->pbuf + off, 0, 3 * off * sizeof(float));
@@ -537,11 +549,13 @@ MSX_API int msx_unet_conv(msx_ctx ctx, int mode, int ks, const float* x, const f
         PackArgs pa{};
         void* buf = nullptr;
         pa.layer[0] = mode == kFwd ? PackLayer{mode, cout, cin, 0, 0} : PackLayer{mode, cin, cout, 0, 0};
-        UCHK(msx_ctx_scratch(ctx, sizeof(__bf16) * conv3_pack_size(pa.layer[0].M, pa.layer[0].C), &buf));
-        pa.w = w;
-        pa.out = static_cast<__bf16*>(buf);
-        UHIP(launch_pack_conv3(pa, 1, msx_ctx_stream(ctx)));
-        a.pack = pa.out;
+        // (the general kernel where there is no room for the packed weights)
+        if (msx_ctx_scratch(ctx, sizeof(__bf16) * conv3_pack_size(pa.layer[0].M, pa.layer[0].C), &buf) == MSX_OK) {
+            pa.w = w;
+            pa.out = static_cast<__bf16*>(buf);
+            UHIP(launch_pack_conv3(pa, 1, msx_ctx_stream(ctx)));
+            a.pack = pa.out;
+        }
     }
     const WgradLayer wl{a, ks};
     hipError_t e = mode == kBwdWeight ? launch_wgrad(&wl, 1, msx_ctx_stream(ctx))
