@@ -816,7 +816,96 @@ __global__ __launch_bounds__(256, SEP && !ADS ? 3 : 2) void rec_sf_kernel(RecArg
         }
 }
 
+// The sum for small potentials: one 16x16 tile of reflections per block, one
+// reflection per thread.  Per chunk of 8 atoms the block evaluates the 16 + 16
+// phase factors of its tile row and column once (one FP64 sincospi per thread)
+// into LDS, and each thread forms the 8 products for its reflection (4 FP64 FMA
+// each).  Every grid index is written, so no clearing goes before it, and its
+// short chunks and 16 times as many work-groups answer sooner where the GPU is not
+// full: the matrix-core kernel walks a slice's atoms 16 at a time with two
+// barriers on a few work-groups (below).
+__device__ __forceinline__ bool refl_index(int i, int n, int mult, int* h) {
+    const int half = n / 2;
+    if (i < half) {
+        *h = i / mult;
+        return i % mult == 0;
+    }
+    const int j = n - i;
+    *h = -(j / mult);
+    return i > half && j % mult == 0;
+}
+
+__global__ __launch_bounds__(256) void rec_sf_point_kernel(RecArgs p) {
+    __shared__ double2 ph[8][32];
+    const int ty = threadIdx.x & 15, tx = threadIdx.x >> 4;
+    const int iy = blockIdx.x * 16 + ty, ix = blockIdx.y * 16 + tx;
+    const int kz = p.kz0 + (int)blockIdx.z;
+    int h, k;
+    const bool ok = refl_index(ix, p.nx, p.nmult, &h) & refl_index(iy, p.ny, p.mmult, &k);
+    const double gx = h * p.A, gy = k * p.B;
+    const double s2 = 0.25 * (gx * gx + gy * gy - 2.0 * gx * gy * p.cg);
+    // this thread's phase-factor slot: atom (tid / 32) of the chunk, column
+    // (tid % 32): 0..15 = h of tile column, 16..31 = k of tile row
+    const int slot_a = threadIdx.x >> 5, slot_c = threadIdx.x & 31;
+    int slot_q;
+    if (slot_c < 16) refl_index(blockIdx.y * 16 + slot_c, p.nx, p.nmult, &slot_q);
+    else refl_index(blockIdx.x * 16 + slot_c - 16, p.ny, p.mmult, &slot_q);
+    double vr = 0.0, vi = 0.0;
+    for (int sg = p.slice_seg[kz]; sg < p.slice_seg[kz + 1]; ++sg) {
+        const RecSeg seg = p.segs[sg];
+        double sr = 0.0, si = 0.0;
+        for (int a0 = seg.start; a0 < seg.end; a0 += 8) {
+            const int ai = a0 + slot_a;
+            if (ai < seg.end) {
+                const RecAtom at = p.atoms[ai];
+                double arg = (double)slot_q * (slot_c < 16 ? at.x : at.y);
+                arg -= rint(arg);
+                double sn, cs;
+                sincospi(-2.0 * arg, &sn, &cs);
+                if (slot_c < 16) {
+                    sn *= at.occ;
+                    cs *= at.occ;
+                }
+                ph[slot_a][slot_c] = make_double2(cs, sn);
+            }
+            __syncthreads();
+            const int na = min(8, seg.end - a0);
+            for (int j = 0; j < na; ++j) {
+                const double2 a = ph[j][tx], b = ph[j][16 + ty];
+                sr = fma(a.x, b.x, fma(-a.y, b.y, sr));
+                si = fma(a.x, b.y, fma(a.y, b.x, si));
+            }
+            __syncthreads();
+        }
+        double f = 0.0;
+        if (p.curves) {
+            curve_at(p.curves + (long long)seg.Z * p.npoints, p.npoints, sqrt(s2) / p.dds, &f);
+        } else {
+            const double* dt = c_dt[seg.Z];
+            for (int j = 0; j < 4; ++j) f += dt[2 * j] * exp(-(dt[2 * j + 1] + seg.dw) * s2);
+            f *= p.inv_area;
+        }
+        vr += f * (sr - seg.ads * si);
+        vi += f * (si + seg.ads * sr);
+    }
+    if (!ok) vr = vi = 0.0;
+    p.out[((long long)blockIdx.z * p.nx + ix) * p.ny + iy] = make_double2(vr, vi);
+}
+
+// From this many grid points times slices the matrix cores are used.  Whole
+// calls, us, reflection per thread / matrix cores, atoms per slice 8, 40, 150, 600 of
+// three species: 64^2 x 4 67 / 74, 72 / 78, 94 / 104, 193 / 244; 256^2 x 4 (256k
+// points) 76 / 81, 84 / 86, 107 / 114, 227 / 240; 384^2 x 4 (576k) 96 / 94, 107 / 99,
+// 149 / 127, 327 / 257; 512^2 x 4 (1M) 111 / 103, 131 / 108, 191 / 136, 468 / 263.
+// Oblique cells and multiples gain the same from 576k on (multiples 92 / 101, 103 /
+// 106, 144 / 133, 321 / 258), and lose up to 26% below.
+constexpr long long kRecTilePoints = 1LL << 19;
+
 hipError_t launch_rec_sf(const RecArgs& a, int nslices, hipStream_t s) {
+    if ((long long)a.nx * a.ny * nslices < kRecTilePoints) {
+        hipLaunchKernelGGL(rec_sf_point_kernel, dim3(a.ny / 16, a.nx / 16, nslices), dim3(256), 0, s, a);
+        return hipGetLastError();
+    }
     const int nrow = rec_count(a.nx, a.nmult), ncol = 2 * rec_count(a.ny, a.mmult);
     if (a.nmult != 1 || a.mmult != 1) {
         // the indices that are no multiple keep zeros
