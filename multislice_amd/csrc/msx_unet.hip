@@ -545,7 +545,10 @@ MSX_API int msx_unet_conv(msx_ctx ctx, int mode, int ks, const float* x, const f
     a.accumulate = 0;
     const size_t need = mode == kBwdWeight ? conv_wgrad_scratch(ks, a) : 0;
     if (need) UHIP(hipMalloc(&a.partial, need * sizeof(float)));
-    if (mode != kBwdWeight && ks == 3 && conv3_fits(a)) {
+    // (packing costs a launch, which fewer than 8 channels do not make up for:
+    // forward 4 channels of 64^2 44.8 / 47.9 us general / packed, 16 of 32^2 53.8 /
+    // 46.9; input gradient 8 of 16^2 51.9 / 50.2)
+    if (mode != kBwdWeight && ks == 3 && conv3_fits(a) && (mode == kFwd ? cin : cout) >= 8) {
         PackArgs pa{};
         void* buf = nullptr;
         pa.layer[0] = mode == kFwd ? PackLayer{mode, cout, cin, 0, 0} : PackLayer{mode, cin, cout, 0, 0};
