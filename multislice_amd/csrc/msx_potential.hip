@@ -584,8 +584,11 @@ __global__ __launch_bounds__(kTileThreads) void splat_tile_kernel(SplatArgs p) {
 // 10 A 877 / 555, of 1 A 166 / 146, of one species 218 / 185, of 20 (192
 // intervals) 244 / 230, of 30 (128) 251 / 251 and of 60 (64) 277 / 298; 2048^2 x
 // 8 519 / 387.  Filling LDS and 4096 wavefronts' worth of larger tiles is what
-// the smaller calls do not make up for.
-constexpr long long kTilePixels = 3LL << 20;
+// the smaller calls do not make up for.  More than 8 species leave fewer intervals
+// of each in LDS and break even later: 512^2 x 12 of 20 species 150 / 166, x 24
+// 200 / 195.
+constexpr long long kTilePixels = 3LL << 20, kTilePixelsMany = 6LL << 20;
+constexpr int kTileFewSpecies = 8;
 constexpr int kTileIntervals = 192;
 
 hipError_t launch_splat(const SplatArgs& args, hipStream_t s) {
@@ -594,7 +597,8 @@ hipError_t launch_splat(const SplatArgs& args, hipStream_t s) {
     a.dy = a.b / a.ny;
     a.bwx = a.a / a.nbx;
     a.bwy = a.b / a.nby;
-    if (a.rtab && (long long)a.nx * a.ny * a.nslices >= kTilePixels && a.nsp <= kSplatInt / kTileIntervals) {
+    const long long least = a.nsp <= kTileFewSpecies ? kTilePixels : kTilePixelsMany;
+    if (a.rtab && (long long)a.nx * a.ny * a.nslices >= least && a.nsp <= kSplatInt / kTileIntervals) {
         const double r2max = a.radius * a.radius;
         int e;
         const double f = std::frexp(r2max, &e);  // r2max = 2 f 2^(e - 1), 2 f in [1, 2)
