@@ -452,7 +452,10 @@ MSX_API int msx_multislice_noalloc(msx_ctx ctx, const msx_stack* stack, const vo
  * group) units from device-side work counters (one per XCD, so that
  * neighbouring column groups stay on one L2).  A tuned grid's FFT plans
  * apply to the batch as to msx_multislice.  Device buffers only (where
- * = MSX_DEVICE); psi0 may be NULL (psi holds the incident wave). */
+ * = MSX_DEVICE); psi0 may be NULL (psi holds the incident wave).  Jobs may
+ * share buffers: every incident wave is read before any result is written where
+ * they overlap; where they do not, each exit wave is written when its job ends,
+ * so a call that returns an error may have written some of them. */
 typedef struct msx_job {
     const msx_stack* stack;
     const void* trans;  /* [nlayer][nx][ny] complex */

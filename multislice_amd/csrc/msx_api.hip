@@ -792,13 +792,13 @@ constexpr int kLoopFlags = 512;           // work-groups of a persistent loop at
 //  A loop costs about 40 us more than two launches before its first slice and
 // gains per slice.  From 8 MiB of waves on it has won at 6 slices (1.00 to 1.47
 // times the sweeps' speed; in FP64 512^2 of 3 waves 0.96, 512 x 256 of 6 0.98),
-// with fewer waves at 16 (256^2 1 wave: 6 slices 0.97, 12 1.00, 16 1.02, 80 1.12; 384 x 128: 1.08, 1.17,
-// 1.23, 1.34; 384 x 512: 0.94, 1.03, 1.01, 1.07).  Where the sweeps are short for
-// the barriers of the team it does not win at all until the waves are larger:
-// FP32 columns of 512 (1 wave of 80 slices: 512 x 128 0.87, x 256 1.00, x 384
-// 0.92, 512^2 1.01; of 4 MiB: 1.00, 1.13, 1.03, 1.08), 128 x 256 (1 to 8 waves
-// 0.94-1.05, 16 waves 1.05; FP64 0.94-1.05, 1.22), FP64 512 x 128 (1.00; of 4 MiB
-// 1.09).
+// with fewer waves at 16 (256^2 1 wave: 6 slices 0.97, 12 1.00, 16 1.02, 80 1.12;
+// 384 x 128: 1.08, 1.17, 1.23, 1.34; 384 x 512: 0.94, 1.03, 1.01, 1.07).  Where the
+// sweeps are short for the barriers of the team it does not win at all until the
+// waves are larger: FP32 columns of 512 (1 wave of 80 slices: 512 x 128 0.87, x
+// 256 1.00, x 384 0.92, 512^2 1.01; of 4 MiB: 1.00, 1.13, 1.03, 1.08), 128 x 256
+// (1 to 8 waves 0.94-1.05, 16 waves 1.05; FP64 0.94-1.05, 1.22), FP64 512 x 128
+// (1.00; of 4 MiB 1.09).
 template <typename C> bool loop_wanted(msx_ctx ctx, int nx, int ny, int nb, int slices) {
     constexpr bool f32 = sizeof(C) == 8;
     const msx_tuning* tu = ctx->tuning(nx, ny, f32 ? MSX_F32 : MSX_F64);
@@ -1861,7 +1861,7 @@ int partial_impl(msx_ctx ctx, const msx_stack* st, const void* trans, const msx_
     batch = std::min(batch, nang);
     // defocus steps per launch of the lens sweeps: as many images of a batch as
     // stay in the last-level cache between the two (a step of few waves leaves
-    // most of the GPU idle: 13 waves of 256^2 at 21 steps with 80 slices before
+    // most of the GPU idle: 21 waves of 256^2 at 21 steps with 80 slices before
     // them: 1820 us per call with a launch pair per step, 1536 with one for all)
     const int nd = (int)off.size();
     int per = (int)std::max(1LL, std::min<long long>(nd, (320LL << 20) / (long long)(sizeof(C) * img) / batch));

@@ -30,7 +30,8 @@ static_assert(!kColAlt || kTc<1> == kTc<0>, "column plan variants share the thre
 template <int PV> constexpr int row_lpw() { return kT<PV> >= 256 ? 1 : 256 / kT<PV>; }
 
 // columns per work-group of the column sweep (coalescing width), bounded by
-// 1024 threads and by an LDS tile of N*(TW+1) complex values
+// MSX_COL_THREADS threads and by N*(TW+1) complex values of at most 80 KB (the
+// LDS tile, padded after every 8 or 16 elements, is at most 72 KB then)
 #ifndef MSX_COL_TW
 #define MSX_COL_TW 16
 #endif
