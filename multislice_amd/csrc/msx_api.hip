@@ -1212,27 +1212,30 @@ int batch_class(msx_ctx ctx, const msx_job* jobs, std::vector<BatchItem>& g, std
     LoopJob<C>* hjb = reinterpret_cast<LoopJob<C>*>(hbase + o_jb);
     const C** hin = reinterpret_cast<const C**>(hbase + o_io);  // incident waves, then exit waves
     C** hout = reinterpret_cast<C**>(hbase + o_io) + nb;
-    loop = loop && !ctx->loop_off;
+    // the loop advances a wave in place: a job whose psi is its incident wave reads
+    // a copy in the wave's slot, which is kept until the loop has ended well
+    bool in_place = false;
+    for (int i = 0; i < nb; i++) in_place |= !jobs[g[i].job].psi0 || jobs[g[i].job].psi0 == jobs[g[i].job].psi;
+    loop = loop && !ctx->loop_off && (!in_place || ctx->wave.ensure(sizeof(C) * img * nb) == MSX_OK);
     for (int i = 0; i < nb; i++) {
         const msx_job& j = jobs[g[i].job];
         hin[i] = static_cast<const C*>(j.psi0 ? j.psi0 : j.psi);
         hout[i] = static_cast<C*>(j.psi);
-        if (loop && hin[i] == hout[i]) {
-            // the loop advances a wave in place: it reads a copy, in the wave's
-            // slot, which is kept until the loop has ended well
-            if (!(loop = ctx->wave.ensure(sizeof(C) * img * nb) == MSX_OK)) continue;
-            C* slot = static_cast<C*>(ctx->wave.p) + i * img;
-            HIPCHK(hipMemcpyAsync(slot, hout[i], sizeof(C) * img, hipMemcpyDeviceToDevice, ctx->stream));
-            hin[i] = slot;
-        }
+        if (loop && hin[i] == hout[i]) hin[i] = static_cast<C*>(ctx->wave.p) + i * img;
         hjb[i] = LoopJob<C>{hout[i], hin[i], g[i].st->nslice, 0};
     }
     HIPCHK(hipMemcpyAsync(dbase, hbase, tot, hipMemcpyHostToDevice, ctx->stream));
+    // direct: the first sweep reads the incident waves and the last ones write the
+    // exit waves where they are
+    const C* const* din = reinterpret_cast<const C* const*>(dbase + o_io);
+    C* const* dout = reinterpret_cast<C* const*>(dbase + o_io) + nb;
     const C* const* dtt = reinterpret_cast<const C* const*>(dbase + o_tt);
     const C* const* dpt = reinterpret_cast<const C* const*>(dbase + o_pt);
     unsigned* dq = reinterpret_cast<unsigned*>(dbase + o_q);
     if (loop) {
         // every job's loop in one kernel, in the job's own buffers
+        if (in_place)
+            HIPCHK(launch_gather_waves<C>(dout, din, static_cast<C*>(ctx->wave.p), nb, img, ctx->stream));
         LoopArgs<C> a;
         std::memset(&a, 0, sizeof a);
         loop_tables(tb, &a);
@@ -1251,10 +1254,6 @@ int batch_class(msx_ctx ctx, const msx_job* jobs, std::vector<BatchItem>& g, std
     // wave slots
     CHK(ctx->wave.ensure(sizeof(C) * img * nb));
     C* w = static_cast<C*>(ctx->wave.p);
-    // direct: the first sweep reads the incident waves and the last ones write the
-    // exit waves where they are
-    const C* const* din = reinterpret_cast<const C* const*>(dbase + o_io);
-    C* const* dout = reinterpret_cast<C* const*>(dbase + o_io) + nb;
     for (int i = 0; i < nb && !direct; i++)
         HIPCHK(hipMemcpyAsync(w + i * img, hin[i], sizeof(C) * img, hipMemcpyDeviceToDevice, ctx->stream));
     const C *twx, *twy;

@@ -284,6 +284,8 @@ hipError_t launch_rs_dt(const RsArgs& a, hipStream_t s);
 // and a copy of nimg 512 x ny images with the column sweep's access pattern
 // (tw adjacent columns per work-group, 32 threads x 16 rows per column, XCD
 // order)
+template <typename C>
+hipError_t launch_gather_waves(C* const* src, const C* const* slot, C* dst, int nb, long long img, hipStream_t s);
 hipError_t launch_stream_copy(const float2* src, float2* dst, long long n, hipStream_t s);
 hipError_t launch_tile_copy(const float2* src, float2* dst, int nimg, int ny, int tw, hipStream_t s);
 hipError_t launch_det_finish(const double* partial, int ndet, int nb, int groups, double w, double* out,

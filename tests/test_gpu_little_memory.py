@@ -1,6 +1,6 @@
 """Calls whose larger workspaces find no room do with the smaller ones, and
 give the same bits: the defocus steps of a partial-coherence image one by one,
-a STEM scan in batches of 256, the surrogate without packed weights and with
+an exit wave in place by the sweeps, a STEM scan in batches of 256, the surrogate without packed weights and with
 the weight gradients of one layer after the other.  Allocations above a limit
 are refused on the host."""
 import ctypes as C
@@ -39,6 +39,21 @@ def test_partial_coherence(ctx, limit):
     got, _, _ = c.partial_coherence(*args)
     c.close()
     assert nd > 2 and bool((got == want).all())
+
+
+def test_exit_wave_in_place(ctx, limit):
+    """The copy that a persistent loop keeps of its incident waves: without room the sweeps run."""
+    import torch
+    n, a, ns = 128, 12.8, 20
+    t = trans(ns, n)
+    want, got = (torch.ones((4, n, n), dtype=torch.complex64, device="cuda") for _ in range(2))
+    ctx.multislice(t, np.full(ns, 2.0), np.arange(ns), want, a, a, KEV)
+    c = msx.Context(0)
+    limit(300000)  # the tables, less than four waves
+    c.multislice(t, np.full(ns, 2.0), np.arange(ns), got, a, a, KEV)
+    assert c.loop_stats() == (0, 0)
+    c.close()
+    assert bool((got == want).all())
 
 
 def test_stem(ctx, limit):
