@@ -486,7 +486,8 @@ typedef struct msx_detector {
  * propagator of each checkpoint slice the detector sums
  *   out[ck][d][p] += weight * sum_{annulus d} |Psi(k)|^2 / (nx*ny)
  * are taken (the fraction of the incident intensity; Musli sums unnormalised
- * values, MSProject.cs:834-838).  Probes run `batch` at a time (0 = choose).
+ * values, MSProject.cs:834-838).  Probes run `batch` at a time (0 = choose: up
+ * to 2 GiB of waves, on grids of powers of two up to 512 up to 320 MiB).
  * pos: host [nprobe][2] (x, y) in Angstrom; checkpoints: host [nck] slice
  * counts 1..nslice, increasing; out: host [nck][ndet][nprobe] doubles,
  * overwritten if accumulate == 0, else added to.  trans per `where`. */
@@ -527,6 +528,8 @@ typedef struct msx_lens {
  * averaged:  image = sum_angles sum_steps w |psi_img|^2 / (nangles sum w).
  * The angle set and step count follow the reference's float arithmetic.
  * sigmaf == 0 images at df alone (the reference divides 0 by 0 there).
+ * The context keeps up to 320 MiB of the steps' images of a batch, fewer steps
+ * where there is no room.
  * image: nx*ny doubles (host or device per `where`, like trans).  nangles
  * and nsteps (may be NULL) receive the number of angles and defocus steps. */
 MSX_API int msx_partial_coherence(msx_ctx ctx, const msx_stack* stack, const void* trans, const msx_lens* lens,
@@ -561,7 +564,9 @@ MSX_API int msx_unet_forward(msx_unet net, const float* x, float* y, int n, int 
 /* loss (may be NULL) and its gradient w.r.t. the packed parameters (grad may be NULL) */
 MSX_API int msx_unet_gradient(msx_unet net, const float* x, const float* target, int n, int h, int w,
                               double* loss, float* grad, int where);
-/* one Adam step (beta1 0.9, beta2 0.999, eps 1e-8) on the batch; loss may be NULL */
+/* one Adam step (beta1 0.9, beta2 0.999, eps 1e-8) on the batch; loss may be NULL.
+ * The network keeps up to 256 MiB (one layer's, if that is more) of partial
+ * weight gradients beside its activations, one layer's where there is no room. */
 MSX_API int msx_unet_train_step(msx_unet net, const float* x, const float* target, int n, int h, int w, float lr,
                                 double* loss, int where);
 /* One convolution of the network's kernels on device buffers (stride 1, zero
